@@ -1543,24 +1543,47 @@ __global__ void __launch_bounds__(256) k_gemm_f32(GemmArgs g) {
   flush_tile<TC, BM, BN, 256, LDC>(g, sC, m0, n0);
 }
 
-// Split-K fold: C = epilogue(sum over splits in order).
-template <typename TC>
-__global__ void k_splitk_reduce(GemmArgs g, int splits) {
-  const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
+// Split-K fold: C = epilogue(sum over splits). Bound by load latency for the small outputs that take many
+// splits (a 128x8 gradient of 128 splits: 4 blocks of one serial chain of loads each took 8 us), so ZG
+// threads share an element: each adds a contiguous range of the splits in order, sixteen loads in
+// flight, and the ranges are added in order through LDS. The order is fixed by the shape.
+template <typename TC, int ZG>
+__global__ void __launch_bounds__(256) k_splitk_reduce(GemmArgs g, int splits) {
+  constexpr int E = 256 / ZG;  // elements per block
+  const int e = threadIdx.x % E, zg = threadIdx.x / E;
+  const long idx = (long)blockIdx.x * E + e;
   const long MN = (long)g.M * g.N;
-  if (idx >= MN) return;
-  // sixteen splits' loads in flight at a time, added in split order
+  const int per = (splits + ZG - 1) / ZG;
+  int z = zg * per;
+  const int zend = min(splits, z + per);
   float s = 0.f;
-  int z = 0;
-  for (; z + 16 <= splits; z += 16) {
-    float v[16];
+  if (idx < MN) {
+    for (; z + 16 <= zend; z += 16) {
+      float v[16];
 #pragma unroll
-    for (int q = 0; q < 16; q++) v[q] = g.ws[(long)(z + q) * MN + idx];
+      for (int q = 0; q < 16; q++) v[q] = g.ws[(long)(z + q) * MN + idx];
 #pragma unroll
-    for (int q = 0; q < 16; q++) s += v[q];
+      for (int q = 0; q < 16; q++) s += v[q];
+    }
+    for (; z < zend; z++) s += g.ws[(long)z * MN + idx];
   }
-  for (; z < splits; z++) s += g.ws[(long)z * MN + idx];
-  epilogue_store<TC>(g, (int)(idx / g.N), (int)(idx % g.N), s);
+  if constexpr (ZG > 1) {
+    __shared__ float sh[ZG][E];
+    sh[zg][e] = s;
+    __syncthreads();
+    if (zg > 0) return;
+#pragma unroll
+    for (int q = 1; q < ZG; q++) s += sh[q][e];
+  }
+  if (idx < MN) epilogue_store<TC>(g, (int)(idx / g.N), (int)(idx % g.N), s);
+}
+// Threads per element: as many as leave each >= 8 splits, while the grid stays within about 2048 blocks.
+template <typename TC>
+void launch_splitk_reduce(const GemmArgs& g, int splits, hipStream_t st) {
+  const long MN = (long)g.M * g.N;
+  if (splits >= 64 && MN <= 32 * 1024) k_splitk_reduce<TC, 16><<<ceil_div(MN, 16), 256, 0, st>>>(g, splits);
+  else if (splits >= 32 && MN <= 128 * 1024) k_splitk_reduce<TC, 4><<<ceil_div(MN, 64), 256, 0, st>>>(g, splits);
+  else k_splitk_reduce<TC, 1><<<ceil_div(MN, 256), 256, 0, st>>>(g, splits);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -1714,11 +1737,11 @@ int pad2d(int dtype, const void* src, long rows, long cols, long ld, int slot, l
 
 // Zero-padded copies of the operands whose contiguous extent, leading dimension, K or base address
 // miss the MFMA kernels' vector preconditions: the contiguous extent and K round up to `vec`. K is
-// padded in both operands (the zeros add nothing to the products); padded rows of A or columns of B
-// feed only output rows and columns that are never stored.
+// padded in both operands (the zeros add nothing to the products) unless neither is k-contiguous;
+// padded rows of A or columns of B feed only output rows and columns that are never stored.
 int pad_operands(PhGemmDesc& d, int vec, hipStream_t st) {
   auto up = [vec](long x) { return (x + vec - 1) / vec * vec; };
-  const long K8 = up(d.K);
+  const long K8 = d.trans_a && !d.trans_b ? d.K : up(d.K);
   const bool padK = K8 != d.K;
   const long a_contig = d.trans_a ? d.M : d.K, b_contig = d.trans_b ? d.K : d.N;
   const bool padA = padK || a_contig % vec || d.lda % vec || ((uintptr_t)d.A % 16);
@@ -1762,14 +1785,18 @@ int gemm(const PhGemmDesc& d_in, hipStream_t st) {
   PH_REQUIRE(d.epi != PH_EPI_RELU_MASK || d.aux, "gemm: mask tensor missing");
 
   // Vector-load preconditions of the MFMA kernels: every 8 (bf16 math) or 4 (fp32 math) consecutive
-  // elements along each operand's contiguous dimension, and along K, start on a multiple of that
-  // count. Shapes that miss them (a 28-wide observation, a 15-wide head) run on zero-padded copies
+  // elements along each operand's contiguous dimension, and along K where an operand is k-contiguous,
+  // start on a multiple of that count. In the TN form (the weight gradients, K = rows of the minibatch)
+  // both operands are loaded by whole k-rows, each checked against the end of the reduction, so any K
+  // runs in place: an odd row count costs no padded copy of the activations, and on an update lane no
+  // scalar kernel (the head's 32x96x6699 fp32 weight gradient 1909 -> 15 us). Other shapes that miss them (a 28-wide observation, a 15-wide head) run on zero-padded copies
   // of the operands. A call with its own workspace slot (a concurrent update lane) takes the scalar
   // kernel instead, as the padded copies live in buffers shared by the calls of the default slot.
   const int vec = d.math == PH_MATH_F32 ? 4 : 8;
   const long a_contig = d.trans_a ? d.M : d.K, b_contig = d.trans_b ? d.K : d.N;
   bool aligned = a_contig % vec == 0 && d.lda % vec == 0 && b_contig % vec == 0 && d.ldb % vec == 0 &&
-                 d.K % vec == 0 && ((uintptr_t)d.A % 16) == 0 && ((uintptr_t)d.B % 16) == 0;
+                 (d.K % vec == 0 || (d.trans_a && !d.trans_b)) && ((uintptr_t)d.A % 16) == 0 &&
+                 ((uintptr_t)d.B % 16) == 0;
   if (!aligned && d.ws_slot <= 0 && d.K > 0) {
     // the padded copies' rows (and K) are whole multiples of vec, whatever the logical M and N
     PH_TRY(pad_operands(d, vec, st));
@@ -1799,6 +1826,7 @@ int gemm(const PhGemmDesc& d_in, hipStream_t st) {
   const long tiles128 = (long)((d.M + 127) / 128) * ((d.N + 127) / 128);
   const long tiles64 = (long)((d.M + 63) / 64) * ((d.N + 63) / 64);
   const bool big_ok = d.math == PH_MATH_BF16 && d.a_dtype == PH_BF16 && d.b_dtype == PH_BF16;
+  const bool f32m = d.math == PH_MATH_F32;
   bool small = false, big = big_ok && tiles256x128 >= 512, wide_n = false;
   // NT outputs at most 64 wide (the policy heads): 256x64 tiles, half the wasted columns of 256x128
   int big_bn = !d.trans_a && d.trans_b && d.N <= 64 ? 64 : 128;
@@ -1818,8 +1846,15 @@ int gemm(const PhGemmDesc& d_in, hipStream_t st) {
       // once the output has >= 16 tiles (512x512x16384: 32 -> 16 splits, 31.8 -> 26.4 us: half the
       // fp32 partials to write and fold)
       const long tw = (long)((d.M + 127) / 128);
-      const long want = big ? 256 / tiles256 : (wide_n ? 256 / tw : (tiles128 >= 16 ? 256 : 512) / tiles128);
-      const long maxs = d.K / (big ? 2048 : 512);
+      // 64x64 splits of >= 256 where 128x128 tiles are mostly padding (an output at most 64 wide or tall
+      // with fp32 operands), or where 128x128 splits of >= 512 leave most CUs idle in fp32 math, whose
+      // tiles are bound by the matrix core (fp32: 128x28x32768 66 -> 13 us, 288x96x6699 74 -> 16 us; bf16 math on
+      // fp32 operands: 128x8x65536 17 -> 10 us)
+      small = !big && !wide_n && (d.a_dtype == PH_F32 || d.b_dtype == PH_F32) &&
+              ((d.M <= 64 || d.N <= 64) || (f32m && tiles128 * (d.K / 512) < 256));
+      const long want = big ? 256 / tiles256
+                            : (wide_n ? 256 / tw : (small ? 256 / tiles64 : (tiles128 >= 16 ? 256 : 512) / tiles128));
+      const long maxs = d.K / (big ? 2048 : (small ? 256 : 512));
       splits = (int)(want < maxs ? want : maxs);
       if (splits < 1) splits = 1;
     } else if (tiles64 >= 128 || d.K < 512) {
@@ -1873,9 +1908,8 @@ int gemm(const PhGemmDesc& d_in, hipStream_t st) {
   }
   PH_LAUNCH_CHECK();
   if (splits > 1) {
-    const long MN = (long)d.M * d.N;
-    if (g.c_bf16) k_splitk_reduce<uint16_t><<<ceil_div(MN, 256), 256, 0, st>>>(g, splits);
-    else k_splitk_reduce<float><<<ceil_div(MN, 256), 256, 0, st>>>(g, splits);
+    if (g.c_bf16) launch_splitk_reduce<uint16_t>(g, splits, st);
+    else launch_splitk_reduce<float>(g, splits, st);
     PH_LAUNCH_CHECK();
   }
   return PH_OK;

@@ -1,0 +1,63 @@
+"""TN products (weight gradients) whose reduction length is no multiple of the vector width: they run in
+place, by whole k-rows, on 64x64 and 128x128 split-K tiles, with a fold of few and of many splits.
+
+The fp32 result is compared with the f64 product of the operands as the kernel reads them: sums of K products
+in fp32, each partial within K 2^-24 relative of the sum of magnitudes; 1e-5 (relative Frobenius) is the
+library's fp32 bar and above the 4e-7 that random signs give."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def D():
+    from pufferlean_amd import device
+    return device
+
+
+@pytest.mark.parametrize("K", [1, 7, 63, 4097, 6699, 33001])
+@pytest.mark.parametrize("M,N", [(8, 8), (32, 96), (136, 40), (288, 96), (64, 520)])
+@pytest.mark.parametrize("dt,math", [("f32", "f32"), ("f32", "bf16"), ("bf16", "bf16")])
+def test_tn_any_k(D, M, N, K, dt, math):
+    g = torch.Generator(device="cuda").manual_seed(K * 1000 + M + N)
+    t = torch.bfloat16 if dt == "bf16" else torch.float32
+    # NaN rows past the end: a read beyond K would poison the sums
+    a = torch.full((K + 8, M), float("nan"), device="cuda", dtype=t)
+    b = torch.full((K + 8, N), float("nan"), device="cuda", dtype=t)
+    a[:K] = torch.randn(K, M, generator=g, device="cuda").to(t)
+    b[:K] = torch.randn(K, N, generator=g, device="cuda").to(t)
+    out = D.gemm(a[:K], b[:K], trans_a=True, math=math)
+    r = (lambda x: x.bfloat16().double()) if math == "bf16" else (lambda x: x.double())
+    ref = r(a[:K]).t() @ r(b[:K])
+    err = ((out.double() - ref).norm() / ref.norm()).item()
+    print(f"TN {M}x{N}x{K} {dt}/{math}: {err:.2e}", flush=True)
+    assert err < 1e-5
+
+
+@pytest.mark.parametrize("B,T", [(7, 13), (45, 31)])
+def test_mingru_gradient_odd_rows(D, B, T):
+    """The head's weight gradient runs on an update lane: an odd row count T*B takes the same kernels as an
+    even one (the gradient of a batch is the sum of its segments' gradients)."""
+    g = torch.Generator(device="cuda").manual_seed(B)
+    Dm, H, L, A = 16, 64, 1, 5
+    kw = dict(precision="f32")
+    cfg = D.MinGRUConfig(B, T, Dm, H, L, A, **kw)
+    one = D.MinGRUConfig(1, T, Dm, H, L, A, **kw)
+    rn = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    p = rn(cfg.P) * 0.1
+    obs, act = rn(T, B, Dm), torch.randint(0, A, (T, B), generator=g, device="cuda", dtype=torch.int32)
+    cols = [rn(T, B) for _ in range(4)]
+    cols[2] = cols[2] * 0.1 - 1.6
+    done = (torch.rand(T, B, generator=g, device="cuda") < 0.1).float()
+    G, _, _ = D.mingru_ppo_grad(cfg, p, obs, act, *cols, done)
+    ref = torch.zeros(cfg.P, device="cuda", dtype=torch.float64)
+    for b in range(B):
+        c = lambda x: x[:, b:b + 1].contiguous()
+        Gb, _, _ = D.mingru_ppo_grad(one, p, c(obs), c(act), *[c(x) for x in cols], c(done))
+        ref += Gb.double()
+    err = ((G.double() - ref).norm() / ref.norm()).item()
+    print(f"mingru odd rows B={B} T={T}: {err:.2e}", flush=True)
+    assert err < 1e-5

@@ -1,10 +1,10 @@
 // V-trace / GAE reverse scan (bandwidth-bound: no MFMA).
 //
-// One lane per segment (two for large fp32 time-major batches) walks t backwards; the recurrence
-// runs in registers with the done mask applied there. Loads are issued a chunk of CH steps ahead of the dependent arithmetic so a lane
-// keeps 4*CH loads in flight. Time-major [T][B] puts consecutive segments on consecutive lanes, so
-// every load and store is a fully coalesced 256 B row per wavefront. Segment-major [B][T] rows are
-// read with 16 B vector loads along t.
+// Large time-major batches ([T][B]): one lane per segment (two for the largest fp32 ones) walks t
+// backwards, the recurrence in registers with the done mask applied there. Loads are issued a chunk of CH
+// steps ahead of the dependent arithmetic so a lane keeps 4*CH loads in flight; consecutive segments on
+// consecutive lanes make every load and store a fully coalesced row per wavefront. Smaller batches and
+// segment-major rows ([B][T]): tiles of segments x steps staged through LDS (k_vtrace_tile).
 //
 // Arithmetic follows the reference's sequential op order with contraction disabled, so the f64
 // kernel is bit-identical to the reference CPU scans (puffercuda.cu:120-132, 200-211) and the f32
@@ -62,19 +62,16 @@ __device__ __forceinline__ void stl(R* p, const Lanes<R, V>& o) {
 // VARIANT 1: bootstrapped form (delta = rho*r + g*V'*nnt - V, V' at T-1 = boot, done := term > .5).
 // rho == nullptr means ratio 1 (plain GAE). Each lane runs the recurrence of V segments side by
 // side, each in the reference's op order.
-template <typename R, int VARIANT, bool TIME_MAJOR, int CH, int V, bool NT>
+template <typename R, int VARIANT, int CH, int V, bool NT>
 __global__ void __launch_bounds__(256) k_vtrace(const R* __restrict__ rew, const R* __restrict__ val,
                                                 const R* __restrict__ term, const R* __restrict__ rho,
                                                 const R* __restrict__ boot, R* __restrict__ adv,
                                                 R* __restrict__ tgt, int B, int T, int rho_is_log,
                                                 int clamp, R gamma, R lam, R rhoClip, R cClip) {
 #pragma clang fp contract(off)
-  static_assert(V == 1 || TIME_MAJOR, "vector lanes run along b (time-major rows)");
   const int b = (blockIdx.x * blockDim.x + threadIdx.x) * V;
   if (b >= B) return;
-  auto at = [&](int t) -> size_t {
-    return TIME_MAJOR ? (size_t)t * (size_t)B + (size_t)b : (size_t)b * (size_t)T + (size_t)t;
-  };
+  auto at = [&](int t) -> size_t { return (size_t)t * (size_t)B + (size_t)b; };
   typedef Lanes<R, V> P;
   const R gl = gamma * lam;
   R last[V], vnext[V];
@@ -174,6 +171,120 @@ __global__ void __launch_bounds__(256) k_vtrace(const R* __restrict__ rew, const
   }
 }
 
+// Workgroup barrier that orders LDS only (loads still in flight are not drained).
+__device__ __forceinline__ void lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Tiled form for batches that do not fill the chip with one lane per segment (a rollout's 4096 segments
+// are 64 wavefronts on 256 CUs, each a chain of dependent load rounds: 13.6 us for 6.3 MB), and for
+// segment-major rows, which lanes would read T elements apart. A block takes SB segments; all 256 threads
+// load a chunk of kTc steps at once, form each step's delta, clipped c and not-done factor in parallel (the
+// ratios' exponentials included), and leave them in LDS; SB lanes then run the recurrence out of LDS, one
+// multiply-multiply-add chain per segment, and all threads write the chunk. The next chunk's loads are in
+// flight during the chain. Same expressions in the same order per element as k_vtrace, so bit-identical.
+// 16 segments a block spread 4096 segments over every CU; neighbouring blocks share cache lines of a
+// time-major row, so each XCD takes a contiguous range of segments. 4096x64: fp32 time-major 12.9 -> 5.7 us,
+// segment-major 60 -> 4.9 (f64 58 -> 6.8); 4096x256 fp32 time-major 46 -> 17.7.
+constexpr int kTc = 64;
+template <typename R, int VARIANT, bool TIME_MAJOR, int SB>
+__global__ void __launch_bounds__(256) k_vtrace_tile(const R* __restrict__ rew, const R* __restrict__ val,
+                                                     const R* __restrict__ term, const R* __restrict__ rho,
+                                                     const R* __restrict__ boot, R* __restrict__ adv,
+                                                     R* __restrict__ tgt, int B, int T, int rho_is_log,
+                                                     int clamp, R gamma, R lam, R rhoClip, R cClip) {
+#pragma clang fp contract(off)
+  constexpr int P = SB + 1, E = SB * kTc / 256;
+  static_assert(E * 256 == SB * kTc, "tile / threads");
+  static_assert((4 * kTc + 1) * P * sizeof(R) <= kMaxLdsBytes, "LDS budget");
+  __shared__ R sV[(kTc + 1) * P], sD[kTc * P], sC[kTc * P], sN[kTc * P];  // sV row kTc: V after the chunk
+  const int tid = threadIdx.x;
+  const int nb = gridDim.x, x = blockIdx.x & 7;
+  const int b0 = (x * (nb >> 3) + min(x, nb & 7) + (int)(blockIdx.x >> 3)) * SB;
+  const R gl = gamma * lam;
+  auto pos = [&](int i, int& tl, int& b) {
+    const int id = tid + i * 256;
+    if (TIME_MAJOR) { tl = id / SB; b = id % SB; }
+    else { tl = id % kTc; b = id / kTc; }
+  };
+  R rr[E], vv[E], dd[E], ww[E];
+  // the chunk's steps are t1 - kTc + tl; a step before 0 or a segment past B re-reads a valid element
+  auto load = [&](int t1) {
+#pragma unroll
+    for (int i = 0; i < E; i++) {
+      int tl, b;
+      pos(i, tl, b);
+      const int t = max(t1 - kTc + tl, 0), bb = min(b0 + b, B - 1);
+      const size_t o = TIME_MAJOR ? (size_t)t * B + bb : (size_t)bb * T + t;
+      rr[i] = rew[o];
+      vv[i] = val[o];
+      dd[i] = term[o];
+      ww[i] = rho ? rho[o] : R(1);
+    }
+  };
+  load(T);
+  R last = R(0);
+  if (tid < SB) sV[kTc * P + tid] = VARIANT == 1 ? boot[min(b0 + tid, B - 1)] : R(0);
+  for (int t1 = T; t1 > 0; t1 -= kTc) {
+#pragma unroll
+    for (int i = 0; i < E; i++) {
+      int tl, b;
+      pos(i, tl, b);
+      sV[tl * P + b] = vv[i];
+    }
+    lds_sync();
+#pragma unroll
+    for (int i = 0; i < E; i++) {
+      int tl, b;
+      pos(i, tl, b);
+      const R vnext = sV[(tl + 1) * P + b], v = vv[i];
+      const R w = ratio_of(ww[i], rho_is_log);
+      const R rh = w < rhoClip ? w : rhoClip;
+      const R cc = w < cClip ? w : cClip;
+      const R r = clamp ? clamp_unit(rr[i]) : rr[i];
+      R nnt, delta, gc = gl * cc;
+      if (VARIANT == 0) {
+        nnt = (dd[i] != R(0)) ? R(0) : R(1);
+        delta = rh * (r + gamma * vnext * nnt - v);
+        if (t1 == T && tl == kTc - 1) delta = gc = nnt = R(0);  // adv[T-1] = 0 in the vec form
+      } else {
+        nnt = (dd[i] > R(0.5)) ? R(0) : R(1);
+        delta = rh * r + gamma * vnext * nnt - v;
+      }
+      sD[tl * P + b] = delta;
+      sC[tl * P + b] = gc;
+      sN[tl * P + b] = nnt;
+    }
+    if (t1 > kTc) load(t1 - kTc);
+    lds_sync();
+    if (tid < SB) {
+      const int tlo = t1 < kTc ? kTc - t1 : 0;
+#pragma unroll 8
+      for (int tl = kTc - 1; tl >= tlo; tl--) {
+        last = sD[tl * P + tid] + sC[tl * P + tid] * last * sN[tl * P + tid];
+        sD[tl * P + tid] = last;
+      }
+      sV[kTc * P + tid] = sV[tid];
+    }
+    lds_sync();
+#pragma unroll
+    for (int i = 0; i < E; i++) {
+      int tl, b;
+      pos(i, tl, b);
+      const int t = t1 - kTc + tl;
+      if (t >= 0 && b0 + b < B) {
+        const size_t o = TIME_MAJOR ? (size_t)t * B + b0 + b : (size_t)(b0 + b) * T + t;
+        const R a = sD[tl * P + b];
+        adv[o] = a;
+        if (tgt) tgt[o] = a + sV[tl * P + b];
+      }
+    }
+    lds_sync();
+  }
+}
+
 template <typename R>
 int launch_vtrace(const R* rew, const R* val, const R* term, const R* rho, const R* boot, size_t B,
                   size_t T, int variant, int time_major, int rho_is_log, int clamp, double gamma,
@@ -187,23 +298,48 @@ int launch_vtrace(const R* rew, const R* val, const R* term, const R* rho, const
   const bool wide = sizeof(R) == 4 && time_major && B % 2 == 0 && B >= 2 * 256 * 256 &&
                     aligned8(rew) && aligned8(val) && aligned8(term) && aligned8(rho) &&
                     aligned8(boot) && aligned8(adv) && aligned8(tgt);
-#define PH_VT(VAR, TM, VV, NT)                                                                     \
-  k_vtrace<R, VAR, TM, CH, VV, NT><<<ceil_div(B / VV, 256), 256, 0, st>>>(                           \
+#define PH_VT(VAR, VV, NT)                                                                         \
+  k_vtrace<R, VAR, CH, VV, NT><<<ceil_div(B / VV, 256), 256, 0, st>>>(                           \
       rew, val, term, rho, boot, adv, tgt, (int)B, (int)T, rho_is_log, clamp, (R)gamma, (R)lam,     \
       (R)rhoClip, (R)cClip)
   if constexpr (sizeof(R) == 4) {
     if (wide) {
-      if (variant == 0) PH_VT(0, true, 2, true);
-      else PH_VT(1, true, 2, true);
+      if (variant == 0) PH_VT(0, 2, true);
+      else PH_VT(1, 2, true);
       PH_LAUNCH_CHECK();
       return PH_OK;
     }
   }
-  if (variant == 0) {
-    if (time_major) PH_VT(0, true, 1, false); else PH_VT(0, false, 1, false);
-  } else {
-    if (time_major) PH_VT(1, true, 1, false); else PH_VT(1, false, 1, false);
+  // Time-major batches of 32768 segments and more fill the chip with one lane per segment (512 wavefronts),
+  // which streams whole rows: 65536x64 fp32 18.6 us against 26.1 tiled (f64 32 / 38), 16384x64 13.7 against
+  // 8.2 (f64 21 / 12). Segment-major rows are always tiled (lanes read T elements apart: 65536x64 213 / 25 us).
+  // Tiles of 16 segments while that gives at most two rounds of blocks per CU, and in f64 (64 would pass the
+  // LDS budget); 64 beyond.
+  if (time_major && B >= 32768) {
+    if (variant == 0) PH_VT(0, 1, false); else PH_VT(1, 1, false);
+    PH_LAUNCH_CHECK();
+    return PH_OK;
   }
+#define PH_VTT(VAR, TM, SB)                                                                                \
+  k_vtrace_tile<R, VAR, TM, SB><<<ceil_div(B, SB), 256, 0, st>>>(rew, val, term, rho, boot, adv, tgt, (int)B, \
+                                                                 (int)T, rho_is_log, clamp, (R)gamma, (R)lam, \
+                                                                 (R)rhoClip, (R)cClip)
+#define PH_VTT_ALL(SB)                                                      \
+  do {                                                                      \
+    if (variant == 0) {                                                     \
+      if (time_major) PH_VTT(0, true, SB); else PH_VTT(0, false, SB);       \
+    } else {                                                                \
+      if (time_major) PH_VTT(1, true, SB); else PH_VTT(1, false, SB);       \
+    }                                                                       \
+  } while (0)
+  if constexpr (sizeof(R) == 4) {
+    if (B > 8192) PH_VTT_ALL(64);
+    else PH_VTT_ALL(16);
+  } else {
+    PH_VTT_ALL(16);
+  }
+#undef PH_VTT_ALL
+#undef PH_VTT
 #undef PH_VT
   PH_LAUNCH_CHECK();
   return PH_OK;

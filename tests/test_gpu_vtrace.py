@@ -158,3 +158,53 @@ def test_full_size_replicated_properties(gpu):
     for r in (0, 17, 63):
         assert torch.equal(adv[:, r * B:(r + 1) * B], one)
     assert torch.equal(tgt, adv + rep(val))
+
+
+@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("time_major", [True, False])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("B,T", [(15, 1), (16, 63), (17, 64), (33, 65), (64, 129), (8192, 3), (8193, 5), (8257, 66),
+                                 (32767, 9), (32768, 9)])
+def test_tiled_scan_bit_exact(gpu, dt, B, T, time_major, variant):
+    """Edges of the tiled scan (16 or 64 segments x chunks of 64 steps) and of the rule that chooses it:
+    bit-identical to the sequential twin in the same precision, terminals on chunk boundaries included."""
+    rew, val, done, logr, boot = _bench_inputs(B, T, seed=0x4800 + T)
+    done = done.reshape((T, B) if time_major else (B, T)).copy()
+    for t in range(0, T, 64):  # a terminal on the first and last step of a chunk, counted from the end
+        for tt in (T - 1 - t, T - 64 - t):
+            if tt >= 0:
+                (done[tt] if time_major else done[:, tt])[::3] = 1.0
+    done = done.ravel()
+    ratio = np.exp(logr.astype(dt))
+    ref, tref = O.vtrace(rew, val, done, ratio, boot, B, T, variant=variant, time_major=time_major, dtype=dt)
+    tt = torch.float32 if dt == np.float32 else torch.float64
+    c = lambda x: _cuda(x, tt).reshape((T, B) if time_major else (B, T))
+    adv, tgt = D.vtrace(c(rew), c(val), c(done), c(ratio), _cuda(boot, tt), variant=variant, time_major=time_major)
+    assert np.array_equal(adv.cpu().numpy().ravel(), ref)
+    if dt == np.float32:
+        assert np.array_equal(tgt.cpu().numpy().ravel(), tref)
+    # in place on the rewards, without targets
+    r = c(rew)
+    D.vtrace(r, c(val), c(done), c(ratio), _cuda(boot, tt), variant=variant, time_major=time_major, out_adv=r,
+             want_targets=False)
+    assert np.array_equal(r.cpu().numpy().ravel(), ref)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float64])
+@pytest.mark.parametrize("n", [1, 2, 255, 4095, 4096, 4097, 8191, 70001])
+@pytest.mark.parametrize("mean", [0.0, 300.0])
+def test_adv_normalize_chunk_edges(gpu, dt, n, mean):
+    """Mean and std of one read in 4096-element chunks, moved to the common mean: against f64. The fp32 mean of
+    n values of size m is off by about m 2^-24 (chunk sums of 16 values per lane and trees), relative to a std of 1;
+    4e-5 covers m = 300 (4 x 300 x 2^-24 = 7e-5 at worst per chunk, averaged over chunks), 1e-12 f64."""
+    x = torch.randn(n, generator=torch.Generator().manual_seed(n), dtype=torch.float64) + mean
+    x = x.to(dt)
+    stats = torch.zeros(2, device="cuda", dtype=dt)
+    y = D.adv_normalize(x.cuda(), stats=stats).double().cpu()
+    xd = x.double()
+    sd = xd.std(unbiased=False) + 1e-8
+    tol = (1e-5 if mean == 0.0 else 8e-5) if dt == torch.float32 else 1e-11
+    if n > 1:
+        assert (y - (xd - xd.mean()) / sd).abs().max().item() <= tol * max(1.0, float(1 / sd))
+        assert abs(stats[1].item() - float(sd)) <= tol * float(sd)
+    assert abs(stats[0].item() - float(xd.mean())) <= tol * max(1.0, mean / 30)

@@ -168,9 +168,9 @@ def ns_set_spin_limit(polls=0):
 
 
 def ns_set_queues(mode=0):
-    """Placement of the fused Newton-Schulz work: 0 by shape (per-XCD queues when every phase of every
-    matrix fits one XCD; the default), 1 one device-wide queue, 2 one queue per XCD. All give
-    bit-identical matrices."""
+    """Placement of the fused Newton-Schulz work: 0 by shape (one workgroup per matrix, one XCD per
+    matrix, or spread over the XCDs; the default), 1 one device-wide queue, 2 one XCD per matrix. All
+    give bit-identical matrices."""
     L.call("ph_ns_set_queues", int(mode))
 
 

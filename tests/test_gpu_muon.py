@@ -207,3 +207,30 @@ def test_ns_wait_failure_is_reported(gpu):
     for m, b in zip(mats, batch):
         ref = O.newton_schulz(m.astype(np.float64), O.BASELINE_COEFFS, 1e-7, form=1)
         assert rel(b.cpu().numpy(), ref) < 1e-2
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (1, 7), (3, 128), (31, 33), (32, 512), (33, 32), (64, 64), (65, 127),
+                                   (96, 160), (128, 4), (128, 128), (100, 128), (160, 96), (512, 5), (129, 128),
+                                   (32, 513), (97, 161)])
+def test_ns_one_workgroup_identical_to_queues(gpu, shape):
+    """A matrix that fits one CU's LDS runs in one workgroup (up to 128x128, 96x160, 32x512 and their
+    transposes; the last three shapes are just past it): bit-identical to the queued launch, alone and in a
+    batch that a large matrix sends to the queues, and within 1e-2 of the f64 iteration."""
+    X0 = rng.normal(0x360 + shape[0] + shape[1], shape[0] * shape[1], 0.0, 0.02).reshape(shape).astype(np.float32)
+    one = torch.from_numpy(X0).cuda()
+    D.newton_schulz(one, coeffs=O.REF_COEFFS, math="bf16")
+    try:
+        D.ns_set_queues(1)
+        q = torch.from_numpy(X0).cuda()
+        D.newton_schulz(q, coeffs=O.REF_COEFFS, math="bf16")
+        D.ns_status()
+    finally:
+        D.ns_set_queues(0)
+    big = torch.from_numpy(rng.normal(0x361, 300 * 300).reshape(300, 300).astype(np.float32)).cuda()
+    mixed = torch.from_numpy(X0).cuda()
+    D.newton_schulz_batch([mixed, big], coeffs=O.REF_COEFFS, math="bf16")
+    D.ns_status()
+    assert torch.equal(one, q)
+    assert torch.equal(one, mixed)
+    ref = O.newton_schulz(X0.astype(np.float64), O.REF_COEFFS, 1e-7, form=1)
+    assert rel(one.cpu().numpy(), ref) < 1e-2

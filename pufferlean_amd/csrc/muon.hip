@@ -530,7 +530,8 @@ int stepvec_exact(long n, const double* b, const double* g, const double* m, dou
 }
 
 // ---- fast tier as a GEMM chain: in-place NS of one fp32 matrix -------------------------------------
-// Used for fp32 MFMA math and for zero steps (normalisation only); bf16 runs fused (ns.hip).
+// Used for fp32 MFMA math past the shapes of the batched launches (ns_f32.hip) and for zero steps
+// (normalisation only); bf16 runs fused (ns.hip).
 // Per step, all operands read straight from fp32 buffers:
 //   A  = X X^T                 (bf16 MFMA; math == PH_MATH_F32: fp32 MFMA)
 //   B  = b A + c A A^T         (split-bf16 MFMA, epilogue b*A + c*acc)
@@ -541,6 +542,8 @@ int newton_schulz_fast(float* X, int rows, int cols, const float* coeffs, int ns
                        int math, int ns_slot, int ws_slot, hipStream_t st) {
   const long n = (long)rows * cols;
   if (n == 0) return PH_OK;
+  if (math == PH_MATH_F32 && nsteps > 0 && ns_f32_fits(rows, cols))
+    return ns_f32_batch(&X, &rows, &cols, 1, coeffs, nsteps, eps, ns_slot, st);
   const int m = rows < cols ? rows : cols, w = rows < cols ? cols : rows;
   const long mm = (long)m * m;
   const long chunk = 4096;
@@ -609,6 +612,25 @@ int muon_fast(float* W, const float* G, float* M, int rows, int cols, float gsca
   return PH_OK;
 }
 
+// The matrices of a batch that the fp32 batched launches take, in groups of kNsMaxMats on st.
+static int ns_f32_fitting(float* const* X, const int* rows, const int* cols, int n, const float* coeffs, int nsteps,
+                          float eps, hipStream_t st) {
+  float* fx[kNsMaxMats];
+  int fr[kNsMaxMats], fc[kNsMaxMats], nf = 0;
+  for (int i = 0; i < n; i++) {
+    if (ns_f32_fits(rows[i], cols[i])) {
+      fx[nf] = X[i];
+      fr[nf] = rows[i];
+      fc[nf++] = cols[i];
+    }
+    if (nf == kNsMaxMats || (nf > 0 && i + 1 == n)) {
+      PH_TRY(ns_f32_batch(fx, fr, fc, nf, coeffs, nsteps, eps, kSlotNs, st));
+      nf = 0;
+    }
+  }
+  return PH_OK;
+}
+
 int muon_fast_batch(const MuonMat* mats, int n, float gscale, float lr, float wd, float mu, float eps,
                     const float* coeffs, int nsteps, int math, hipStream_t st) {
   if (n <= 0) return PH_OK;
@@ -647,8 +669,12 @@ int muon_fast_batch(const MuonMat* mats, int n, float gscale, float lr, float wd
     PH_LAUNCH_CHECK();
   }
   if (math == PH_MATH_F32 || nsteps == 0) {
-    for (int i = 0; i < n; i++)
+    const bool batched = math == PH_MATH_F32 && nsteps > 0;
+    if (batched) PH_TRY(ns_f32_fitting(X, rows, cols, n, coeffs, nsteps, eps, st));
+    for (int i = 0; i < n; i++) {
+      if (batched && ns_f32_fits(rows[i], cols[i])) continue;
       PH_TRY(newton_schulz_fast(X[i], rows[i], cols[i], coeffs, nsteps, eps, math, kSlotNs, 0, st));
+    }
   } else {
     PH_TRY(ns_fused(X, rows, cols, n, coeffs, nsteps, eps, kSlotNs, kSlotNsCtl, st));
   }
@@ -740,15 +766,23 @@ extern "C" int ph_newton_schulz_batch(float* const* X, const int* rows, const in
   // bf16: the whole batch in fused launches on `stream`
   if (math != PH_MATH_F32 && nsteps > 0)
     return ns_fused(X, rows, cols, n, coeffs, nsteps, eps, kSlotNs, kSlotNsCtl, st);
-  // fp32 MFMA: matrix i runs on stream lane i % kLanes with that lane's scratch; the lanes fork
-  // from and join back into `stream`.
-  const int nl = n < kLanes ? n : kLanes;
+  // fp32 MFMA: the matrices that fit share launches on `stream`
+  const bool batched = math == PH_MATH_F32 && nsteps > 0;
+  if (batched) PH_TRY(ns_f32_fitting(X, rows, cols, n, coeffs, nsteps, eps, st));
+  const auto rest = [&](int i) { return !batched || !ns_f32_fits(rows[i], cols[i]); };
+  int left = 0;
+  for (int i = 0; i < n; i++) left += rest(i);
+  if (left == 0) return PH_OK;
+  // the others run on stream lanes, the i-th on lane i % kLanes with that lane's scratch; the lanes fork from
+  // and join back into `stream`
   LaneJoin lanes(st);
-  PH_TRY(lanes.fork(nl));
-  for (int i = 0; i < n; i++) {
-    const LaneSlots sl = lane_slots(i % kLanes);
+  PH_TRY(lanes.fork(left < kLanes ? left : kLanes));
+  for (int i = 0, q = 0; i < n; i++) {
+    if (!rest(i)) continue;
+    const int lane = q++ % kLanes;
+    const LaneSlots sl = lane_slots(lane);
     PH_TRY(newton_schulz_fast(X[i], rows[i], cols[i], coeffs, nsteps, eps, math, sl.ns, sl.gemm_ws,
-                              lane_stream(i % kLanes)));
+                              lane_stream(lane)));
   }
   return lanes.join();
 }

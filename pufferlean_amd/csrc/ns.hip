@@ -48,10 +48,10 @@
 // (the XCC_ID hardware register). Matrices whose phases all fit one XCD (at most 32 tiles) are pinned to one
 // queue each (largest estimated work first, each to the least loaded queue): their items, iterates and
 // products stay on that XCD and the data moves through its L2 (plain stores, L2 hits; every line a block
-// reads was written earlier in the launch by a block of the same XCD). Otherwise every phase's items are
-// dealt to the queues in contiguous ranges (P3's column by column), so that an XCD's tiles share operand
-// rows in its L2, with device-coherent (write-through) stores; six matrices of 512 rows 326 -> 294 us against
-// one device-wide queue with a k loop per product. Other devices take that one queue. Control words are
+// reads was written earlier in the launch by a block of the same XCD). Otherwise, where a P3 has at most one
+// item per CU, every phase's items are dealt to the queues in contiguous ranges (P3's column by column), so
+// that an XCD's tiles share operand rows in its L2, with device-coherent (write-through) stores. Larger
+// batches and other devices take one device-wide queue. Control words are
 // device-scope in all of them (atomics, and relaxed device-scope loads for polling; many blocks poll one
 // word, and polling with atomics serialises them behind the signal they wait for). Measured (5 steps)
 // pinned against one device-wide queue: 64x64 103 us against 139, 128x128 119 against 164, but 512x512 425
@@ -983,7 +983,8 @@ int ns_fused(float* const* X, const int* rows, const int* cols, int n, const flo
   PH_TRY(ensure_zeroed_words(ctl, kCtlWords, st));
   // On a device of kNsQueues XCDs of kXcdCus CUs: matrices pinned to one XCD each when every phase of
   // every matrix fits it (one block per CU, so kXcdCus tiles at a time), else every phase's items spread
-  // over the XCDs' queues in contiguous ranges. Elsewhere, and in mode 1, one device-wide queue.
+  // over the XCDs' queues in contiguous ranges, or in one device-wide queue (below). Elsewhere, and in mode
+  // 1, one device-wide queue.
   const int cus = cu_count();
   const bool xcds = mode != 1 && cus == kNsQueues * kXcdCus;
   bool local = xcds;
@@ -1024,7 +1025,14 @@ int ns_fused(float* const* X, const int* rows, const int* cols, int n, const flo
     unsigned char* ws = (unsigned char*)scratch(ws_slot, bytes);
     if (!ws) return PH_ERR_NOMEM;
     for (int k = 0; k < L.nmat; k++) L.mat[k].ws = ws + (uintptr_t)L.mat[k].ws;
-    L.nq = xcds ? kNsQueues : 1;
+    // A phase with more items than CUs takes several rounds, and fixed shares leave some XCDs a round more
+    // than others while a shared queue evens them out; one that fits the chip gains from shared operand
+    // panels (per-XCD ranges against one queue: two 1536x512 322 against 292 us, six of 512 rows 296 / 278,
+    // two 768x768 350 / 317; but 1536x512 254 / 285, four 512x512 217 / 228, 768x768 287 / 308).
+    long c3 = 0;
+    for (int k = 0; k < L.nmat; k++) c3 += n3[k];
+    const bool split = xcds && (local || c3 <= cus);
+    L.nq = split ? kNsQueues : 1;
     if (local) {
       // matrices to queues: largest estimated work first, each to the least loaded queue (ties: the lower
       // index); the list is then ordered by queue (a queue's matrices in their given order), so that each
@@ -1087,7 +1095,7 @@ int ns_fused(float* const* X, const int* rows, const int* cols, int n, const flo
     // bandwidth goes to one tile at a time). Per-XCD queues take every CU (a queue with no items releases
     // its blocks at once).
     const long cap = cus;
-    const unsigned grid = xcds ? (unsigned)cap : (unsigned)(total < cap ? total : cap);
+    const unsigned grid = split ? (unsigned)cap : (unsigned)(total < cap ? total : cap);
     L.qmask = 0u;
     for (int q = 0; q < L.nq; q++)
       if (L.i0.qlo[q + 1] > L.i0.qlo[q] || L.it.qlo[q + 1] > L.it.qlo[q] || L.i3.qlo[q + 1] > L.i3.qlo[q])

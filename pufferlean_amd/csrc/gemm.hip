@@ -1789,9 +1789,10 @@ int gemm(const PhGemmDesc& d_in, hipStream_t st) {
   // start on a multiple of that count. In the TN form (the weight gradients, K = rows of the minibatch)
   // both operands are loaded by whole k-rows, each checked against the end of the reduction, so any K
   // runs in place: an odd row count costs no padded copy of the activations, and on an update lane no
-  // scalar kernel (the head's 32x96x6699 fp32 weight gradient 1909 -> 15 us). Other shapes that miss them (a 28-wide observation, a 15-wide head) run on zero-padded copies
-  // of the operands. A call with its own workspace slot (a concurrent update lane) takes the scalar
-  // kernel instead, as the padded copies live in buffers shared by the calls of the default slot.
+  // scalar kernel (the head's 32x96x6699 fp32 weight gradient 1909 -> 15 us). Other shapes that miss them (a
+  // 28-wide observation, a 15-wide head) run on zero-padded copies of the operands. A call with its own
+  // workspace slot (a concurrent update lane) takes the scalar kernel instead, as the padded copies live in
+  // buffers shared by the calls of the default slot.
   const int vec = d.math == PH_MATH_F32 ? 4 : 8;
   const long a_contig = d.trans_a ? d.M : d.K, b_contig = d.trans_b ? d.K : d.N;
   bool aligned = a_contig % vec == 0 && d.lda % vec == 0 && b_contig % vec == 0 && d.ldb % vec == 0 &&

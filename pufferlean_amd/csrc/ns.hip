@@ -39,10 +39,13 @@
 //
 // Scheduling: every tile of every phase of every matrix is one work item with a ticket number in
 // its matrix's queue, ordered by (step, phase, matrix, tile). An item waits only for the items of
-// its matrix in earlier phases, i.e. for smaller tickets of the same queue. A queue's blocks take its
-// tickets from an atomic counter in increasing order, so every item waited on has been taken by a
-// block that is already running (or runs an earlier item of its own): the launch completes for any grid
-// size, without assuming that all blocks are co-resident. The launch's last block to leave resets the counters for the next launch.
+// its matrix in earlier phases: smaller tickets of the same queue, or, where phases are spread over the
+// XCDs' queues, items of earlier phases there. A queue's blocks take its tickets from an atomic counter in
+// increasing order. On one queue, or with matrices pinned to one each, every item waited on has therefore been
+// taken by a block that is already running (or runs an earlier item of its own), and the launch completes for
+// any grid size. Spread phases need a block on every XCD with work, which the grid of one block per CU
+// gives once the work before it has left the XCD; an unfinished item of the earliest phase is always
+// runnable. Waits are bounded in all of them. The launch's last block to leave resets the counters.
 //
 // Queues: on a device of 8 XCDs of 32 CUs (MI355X), one queue per XCD, served by the blocks that run on it
 // (the XCC_ID hardware register). Matrices whose phases all fit one XCD (at most 32 tiles) are pinned to one
@@ -921,8 +924,8 @@ int ns_small(float* const* X, const int* rows, const int* cols, int n, const flo
 }
 
 std::atomic<unsigned> g_spin{kSpinLimit};
-// 0: per-XCD queues where the device has 8 XCDs of 32 CUs and every phase of every matrix fits one
-// XCD's CUs; 1: always one device-wide queue; 2: per-XCD queues whenever the device has them
+// 0: by shape (one workgroup per matrix, one XCD per matrix, tiles spread over the XCDs, or one device-wide
+// queue); 1: always one device-wide queue; 2: one XCD per matrix whenever the device has 8 XCDs of 32 CUs
 std::atomic<int> g_queues{0};
 
 __global__ void k_clear_word(unsigned* w) {

@@ -425,8 +425,8 @@ __global__ void __launch_bounds__(kGaThreads) k_mb_stats(const double* __restric
 }
 
 // adv[j] = mp[bi] * (adv[j] - mean) / (std + 1e-8), j = t*B + bi (mp NULL: weight 1). FOLD: every block merges
-// the gather's partials itself (up to kFoldMax of them: the merge costs less than a launch of one block: 4.0 + 2.8 -> 4.9 us), and the
-// first writes stats; else stats are given.
+// the gather's partials itself (up to kFoldMax of them: the merge costs less than a launch of one block:
+// 4.0 + 2.8 -> 4.9 us), and the first writes stats; else stats are given.
 template <typename R, bool FOLD>
 __global__ void __launch_bounds__(kGaThreads) k_mb_normalize(R* __restrict__ adv, long B, long n,
                                                              const double* __restrict__ mp,

@@ -208,10 +208,10 @@ int ph_ns_set_spin_limit(unsigned polls);
  * memory (at most sixteen 32x32 tiles: 128x128, 32x512) runs one workgroup per matrix, with no waits between
  * workgroups; else, on a device of 8 XCDs of 32 CUs (MI355X), each matrix runs on the CUs of one XCD, its
  * signals and data in that XCD's L2, when every phase of every matrix has at most 32 output tiles of 64x64
- * (min(rows, cols) <= 256 or so); otherwise a batch whose widest phase has at most one tile per CU is spread
- * over per-XCD queues, and a larger one takes one device-wide queue, with signals and data through memory.
- * 1: always one device-wide queue; 2: each matrix on one XCD whenever the device has them. All give bit-identical matrices. A queue with work but no workgroups on its XCD is recorded, and
- * ph_ns_status reports it. No counterpart in the reference. */
+ * (min(rows, cols) <= 256 or so); otherwise one device-wide queue, with signals and data through memory.
+ * 1: always the device-wide queue; 2: each matrix on one XCD whenever the device has them. All give
+ * bit-identical matrices. A queue with work but no workgroups on its XCD is recorded, and ph_ns_status
+ * reports it. No counterpart in the reference. */
 int ph_ns_set_queues(int mode);
 /* In-place Muon matrix step on fp32 state: M <- mu*M + gscale*G; U = gscale*G + mu*M;
  * W <- (1-lr*wd)*W + lr*sqrt(max(1,rows/cols))*NS(U). */

@@ -1,6 +1,7 @@
 // Internal (non-exported) launch helpers shared between translation units.
 #pragma once
 #include "common.hpp"
+#include "ns_plan.hpp"
 
 namespace ph {
 
@@ -153,7 +154,6 @@ int muon_fast(float* W, const float* G, float* M, int rows, int cols, float gsca
 // launches on `st`): X[i] (rows[i] x cols[i], fp32) is normalised and orthogonalised in place.
 // ws_slot holds the per-matrix, per-step iterates and products (ns_fused_ws_bytes per matrix),
 // ctl_slot the launch's work-item counters; two calls that overlap in time must not share either.
-constexpr int kNsMaxMats = 16;
 constexpr int kNsMaxSteps = 64;
 int ns_fused(float* const* X, const int* rows, const int* cols, int n, const float* coeffs, int nsteps,
              float eps, int ws_slot, int ctl_slot, hipStream_t st);

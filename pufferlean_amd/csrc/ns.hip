@@ -39,27 +39,22 @@
 //
 // Scheduling: every tile of every phase of every matrix is one work item with a ticket number in
 // its matrix's queue, ordered by (step, phase, matrix, tile). An item waits only for the items of
-// its matrix in earlier phases: smaller tickets of the same queue, or, where phases are spread over the
-// XCDs' queues, items of earlier phases there. A queue's blocks take its tickets from an atomic counter in
-// increasing order. On one queue, or with matrices pinned to one each, every item waited on has therefore been
-// taken by a block that is already running (or runs an earlier item of its own), and the launch completes for
-// any grid size. Spread phases need a block on every XCD with work, which the grid of one block per CU
-// gives once the work before it has left the XCD; an unfinished item of the earliest phase is always
-// runnable. Waits are bounded in all of them. The launch's last block to leave resets the counters.
+// its matrix in earlier phases, all of them smaller tickets of the same queue. A queue's blocks take
+// its tickets from an atomic counter in increasing order, so every item waited on has been taken by
+// a block that is already running (or runs an earlier item of its own), and the launch completes for any
+// grid size. Waits are bounded all the same. The launch's last block to leave resets the counters.
 //
-// Queues: on a device of 8 XCDs of 32 CUs (MI355X), one queue per XCD, served by the blocks that run on it
-// (the XCC_ID hardware register). Matrices whose phases all fit one XCD (at most 32 tiles) are pinned to one
-// queue each (largest estimated work first, each to the least loaded queue): their items, iterates and
-// products stay on that XCD and the data moves through its L2 (plain stores, L2 hits; every line a block
-// reads was written earlier in the launch by a block of the same XCD). Otherwise, where a P3 has at most one
-// item per CU, every phase's items are dealt to the queues in contiguous ranges (P3's column by column), so
-// that an XCD's tiles share operand rows in its L2, with device-coherent (write-through) stores. Larger
-// batches and other devices take one device-wide queue. Control words are
-// device-scope in all of them (atomics, and relaxed device-scope loads for polling; many blocks poll one
-// word, and polling with atomics serialises them behind the signal they wait for). Measured (5 steps)
-// pinned against one device-wide queue: 64x64 103 us against 139, 128x128 119 against 164, but 512x512 425
-// against 260 and 1536x512 808 against 303, hence the rule. The launch's last block checks that every queue
-// with work had blocks on its XCD, else it raises a sticky flag that ph_ns_status reports.
+// Queues (ns_plan.hpp): on a device of 8 XCDs of 32 CUs (MI355X), one queue per XCD, served by the blocks that
+// run on it (the XCC_ID hardware register), when every phase of every matrix fits one XCD (at most 32 tiles).
+// Each matrix is pinned to one queue: its items, iterates and products stay on that XCD and the data moves
+// through its L2 (plain stores, L2 hits; every line a block reads was written earlier in the launch by a
+// block of the same XCD). Larger matrices and other devices take one device-wide queue, with
+// device-coherent (write-through) stores. Control words are device-scope in both (atomics, and relaxed
+// device-scope loads for polling; many blocks poll one word, and polling with atomics serialises them behind
+// the signal they wait for). Measured (5 steps), pinned against device-wide: 200x129 119 us against
+// 143, 256x256 125 / 155, 320x320 142 / 183, but 512x512 300 / 219 and 1536x512 592 / 287, hence the rule. The
+// launch's last block checks that every queue with work had blocks on its XCD, else it raises a sticky
+// flag that ph_ns_status reports.
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -91,9 +86,6 @@ struct NsMat {
   int rows, cols;
 };
 
-constexpr int kNsQueues = 8;  // one work queue per XCD
-constexpr int kXcdCus = 32;   // CUs per XCD
-
 // Control words, each polled or updated on its own 128-byte line (32 words): the launch's blocks
 // finished; the wait limit hit in this launch (kCtlFlag; +1: ever hit, +2: a queue with work had no
 // blocks on its XCD, both never cleared by the kernel); the XCDs that had blocks in this launch (bit
@@ -105,13 +97,6 @@ constexpr int kCtlSeen = 2 * kCtlStride;
 constexpr int kCtlTicket = 3 * kCtlStride;                    // + kCtlStride * q
 constexpr int kCtlDone = kCtlTicket + kCtlStride * kNsQueues;  // + kCtlStride * matrix
 constexpr int kCtlWords = kCtlDone + kCtlStride * kNsMaxMats;
-
-// A launch's items of one phase kind (P0; P1 and P2; P3) are numbered through its matrices in list order:
-// matrix k owns [cum[k], cum[k + 1]). Queue q takes the contiguous range [qlo[q], qlo[q + 1]).
-struct NsItems {
-  int cum[kNsMaxMats + 1];
-  int qlo[kNsQueues + 1];
-};
 
 struct NsLaunch {
   NsMat mat[kNsMaxMats];
@@ -438,8 +423,8 @@ __device__ __forceinline__ void p3_store(const NsMat& mt, const Geo& g, long xs,
   }
 }
 
-// LOCAL: every matrix's items run on one XCD (plain stores); otherwise device-coherent stores. With several
-// queues, a block serves the queue of the XCD it runs on.
+// LOCAL: every matrix's items run on one XCD (plain stores), a block serving the queue of the XCD it runs on;
+// otherwise one device-wide queue and device-coherent stores.
 template <bool LOCAL>
 __global__ void __launch_bounds__(kThreads) k_ns_fused(const NsLaunch L) {
   // the two k-groups' double-buffered panels; the epilogue's fold and P0's staging reuse them
@@ -503,8 +488,7 @@ __global__ void __launch_bounds__(kThreads) k_ns_fused(const NsLaunch L) {
     int ti, tj;
     TileOps op;
     if (p == 3) {
-      // column by column: a contiguous share of the tiles then reads few columns of X^T and, as m <= w, at
-      // most all of B'
+      // column by column: blocks that run side by side share rows of X^T and, as m <= w, read at most all of B'
       tj = r / g.tm;
       ti = r - tj * g.tm;
       op.ld = g.mp;
@@ -924,8 +908,7 @@ int ns_small(float* const* X, const int* rows, const int* cols, int n, const flo
 }
 
 std::atomic<unsigned> g_spin{kSpinLimit};
-// 0: by shape (one workgroup per matrix, one XCD per matrix, tiles spread over the XCDs, or one device-wide
-// queue); 1: always one device-wide queue; 2: one XCD per matrix whenever the device has 8 XCDs of 32 CUs
+// 0: by shape (one workgroup per matrix, one XCD per matrix, or one device-wide queue); 1: always one device-wide queue; 2: one XCD per matrix whenever the device has 8 XCDs of 32 CUs
 std::atomic<int> g_queues{0};
 
 __global__ void k_clear_word(unsigned* w) {
@@ -942,25 +925,6 @@ int cu_count() {
     n[dev] = v;
   }
   return n[dev];
-}
-
-// Numbers the launch's items through its matrices (cum of each phase kind); false (with an error) if a
-// queue's tickets could pass 31 bits.
-bool number_items(NsLaunch& L, const long* n0, const long* nt, const long* n3, int nsteps) {
-  long c0 = 0, ct = 0, c3 = 0;
-  for (int k = 0; k < L.nmat; k++) {
-    c0 += n0[k];
-    ct += nt[k];
-    c3 += n3[k];
-    if (c0 + (long)nsteps * (2 * ct + c3) >= (1L << 31)) {
-      set_error("newton_schulz (fused): batch too large");
-      return false;
-    }
-    L.i0.cum[k + 1] = (int)c0;
-    L.it.cum[k + 1] = (int)ct;
-    L.i3.cum[k + 1] = (int)c3;
-  }
-  return true;
 }
 
 }  // namespace
@@ -984,13 +948,11 @@ int ns_fused(float* const* X, const int* rows, const int* cols, int n, const flo
   unsigned* ctl = (unsigned*)scratch(ctl_slot, kCtlWords * 4);
   if (!ctl) return PH_ERR_NOMEM;
   PH_TRY(ensure_zeroed_words(ctl, kCtlWords, st));
-  // On a device of kNsQueues XCDs of kXcdCus CUs: matrices pinned to one XCD each when every phase of
-  // every matrix fits it (one block per CU, so kXcdCus tiles at a time), else every phase's items spread
-  // over the XCDs' queues in contiguous ranges, or in one device-wide queue (below). Elsewhere, and in mode
-  // 1, one device-wide queue.
+  // On a device of kNsQueues XCDs of kXcdCus CUs: matrices pinned to one XCD each when every phase of every
+  // matrix fits it (one block per CU, so kXcdCus tiles at a time). Otherwise, and in mode 1, one device-wide
+  // queue.
   const int cus = cu_count();
-  const bool xcds = mode != 1 && cus == kNsQueues * kXcdCus;
-  bool local = xcds;
+  bool local = mode != 1 && cus == kNsQueues * kXcdCus;
   if (local && mode == 0)
     for (int j = 0; j < n; j++) {
       Geo g;
@@ -1002,13 +964,13 @@ int ns_fused(float* const* X, const int* rows, const int* cols, int n, const flo
     // next group of at most kNsMaxMats non-empty matrices
     NsLaunch L{};
     size_t bytes = 0;
-    long work[kNsMaxMats];
-    long n0[kNsMaxMats], nt[kNsMaxMats], n3[kNsMaxMats];
+    NsMat mats[kNsMaxMats];
+    NsLoad load[kNsMaxMats];
     int j = i;
     for (; j < n && L.nmat < kNsMaxMats; j++) {
       if ((long)rows[j] * cols[j] == 0) continue;
       const int k = L.nmat++;
-      NsMat& m = L.mat[k];
+      NsMat& m = mats[k];
       m.x = X[j];
       m.rows = rows[j];
       m.cols = cols[j];
@@ -1016,78 +978,27 @@ int ns_fused(float* const* X, const int* rows, const int* cols, int n, const flo
       const size_t b = ns_layout(rows[j], cols[j], nsteps, nullptr, g);
       m.ws = (unsigned char*)(uintptr_t)bytes;  // offset for now
       bytes += b;
-      n0[k] = g.n0;
-      nt[k] = g.nt;
-      n3[k] = g.n3;
       // tile-chunk products of a step: P1 over w, P2 three over m, P3 three over m
       const long cw = g.wp / kT, cm = g.mp / kT;
-      work[k] = g.n0 + (long)nsteps * (g.nt * cw + 3 * g.nt * cm + 3 * g.n3 * cm);
+      load[k] = NsLoad{g.n0, g.nt, g.n3, g.n0 + (long)nsteps * (g.nt * cw + 3 * g.nt * cm + 3 * g.n3 * cm)};
     }
     i = j;
     if (L.nmat == 0) continue;
     unsigned char* ws = (unsigned char*)scratch(ws_slot, bytes);
     if (!ws) return PH_ERR_NOMEM;
-    for (int k = 0; k < L.nmat; k++) L.mat[k].ws = ws + (uintptr_t)L.mat[k].ws;
-    // A phase with more items than CUs takes several rounds, and fixed shares leave some XCDs a round more
-    // than others while a shared queue evens them out; one that fits the chip gains from shared operand
-    // panels (per-XCD ranges against one queue: two 1536x512 322 against 292 us, six of 512 rows 296 / 278,
-    // two 768x768 350 / 317; but 1536x512 254 / 285, four 512x512 217 / 228, 768x768 287 / 308).
-    long c3 = 0;
-    for (int k = 0; k < L.nmat; k++) c3 += n3[k];
-    const bool split = xcds && (local || c3 <= cus);
-    L.nq = split ? kNsQueues : 1;
-    if (local) {
-      // matrices to queues: largest estimated work first, each to the least loaded queue (ties: the lower
-      // index); the list is then ordered by queue (a queue's matrices in their given order), so that each
-      // queue's items are a contiguous range
-      int qof[kNsMaxMats], order[kNsMaxMats];
-      for (int k = 0; k < L.nmat; k++) order[k] = k;
-      for (int a = 1; a < L.nmat; a++)  // stable insertion sort by work, descending
-        for (int b = a; b > 0 && work[order[b]] > work[order[b - 1]]; b--) std::swap(order[b], order[b - 1]);
-      long load[kNsQueues] = {};
-      for (int a = 0; a < L.nmat; a++) {
-        int best = 0;
-        for (int q = 1; q < L.nq; q++)
-          if (load[q] < load[best]) best = q;
-        qof[order[a]] = best;
-        load[best] += work[order[a]];
-      }
-      NsMat lm[kNsMaxMats];
-      long l0[kNsMaxMats], lt[kNsMaxMats], l3[kNsMaxMats];
-      int k2 = 0, first[kNsQueues + 1];
-      for (int q = 0; q < L.nq; q++) {
-        first[q] = k2;
-        for (int k = 0; k < L.nmat; k++)
-          if (qof[k] == q) {
-            lm[k2] = L.mat[k];
-            l0[k2] = n0[k];
-            lt[k2] = nt[k];
-            l3[k2++] = n3[k];
-          }
-      }
-      first[L.nq] = k2;
-      for (int k = 0; k < L.nmat; k++) {
-        L.mat[k] = lm[k];
-        n0[k] = l0[k];
-        nt[k] = lt[k];
-        n3[k] = l3[k];
-      }
-      if (!number_items(L, n0, nt, n3, nsteps)) return PH_ERR_UNSUPPORTED;
-      for (int q = 0; q <= L.nq; q++) {
-        L.i0.qlo[q] = L.i0.cum[first[q]];
-        L.it.qlo[q] = L.it.cum[first[q]];
-        L.i3.qlo[q] = L.i3.cum[first[q]];
-      }
-    } else {
-      if (!number_items(L, n0, nt, n3, nsteps)) return PH_ERR_UNSUPPORTED;
-      // equal shares of every phase (the one queue takes all): neighbouring tiles of a matrix share their
-      // operand rows, so an XCD fetches few panels into its L2
-      for (int q = 0; q <= L.nq; q++) {
-        L.i0.qlo[q] = (int)((long)L.i0.cum[L.nmat] * q / L.nq);
-        L.it.qlo[q] = (int)((long)L.it.cum[L.nmat] * q / L.nq);
-        L.i3.qlo[q] = (int)((long)L.i3.cum[L.nmat] * q / L.nq);
-      }
+    NsPlan plan;
+    if (!ns_place(load, L.nmat, nsteps, local, plan)) {
+      set_error("newton_schulz (fused): batch too large");
+      return PH_ERR_UNSUPPORTED;
     }
+    for (int k = 0; k < L.nmat; k++) {
+      L.mat[k] = mats[plan.order[k]];
+      L.mat[k].ws = ws + (uintptr_t)L.mat[k].ws;
+    }
+    L.i0 = plan.i0;
+    L.it = plan.it;
+    L.i3 = plan.i3;
+    L.nq = plan.nq;
     const long total = (long)L.i0.cum[L.nmat] + (long)nsteps * (2L * L.it.cum[L.nmat] + L.i3.cum[L.nmat]);
     for (int k = 0; k < 3 * nsteps; k++) L.coef[k] = coeffs[k];
     L.ctl = ctl;
@@ -1098,7 +1009,7 @@ int ns_fused(float* const* X, const int* rows, const int* cols, int n, const flo
     // bandwidth goes to one tile at a time). Per-XCD queues take every CU (a queue with no items releases
     // its blocks at once).
     const long cap = cus;
-    const unsigned grid = split ? (unsigned)cap : (unsigned)(total < cap ? total : cap);
+    const unsigned grid = local ? (unsigned)cap : (unsigned)(total < cap ? total : cap);
     L.qmask = 0u;
     for (int q = 0; q < L.nq; q++)
       if (L.i0.qlo[q + 1] > L.i0.qlo[q] || L.it.qlo[q + 1] > L.it.qlo[q] || L.i3.qlo[q + 1] > L.i3.qlo[q])

@@ -169,7 +169,7 @@ def ns_set_spin_limit(polls=0):
 
 def ns_set_queues(mode=0):
     """Placement of the fused Newton-Schulz work: 0 by shape (one workgroup per matrix, one XCD per
-    matrix, or spread over the XCDs; the default), 1 one device-wide queue, 2 one XCD per matrix. All
+    matrix, or one device-wide queue; the default), 1 one device-wide queue, 2 one XCD per matrix. All
     give bit-identical matrices."""
     L.call("ph_ns_set_queues", int(mode))
 

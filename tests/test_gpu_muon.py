@@ -209,6 +209,36 @@ def test_ns_wait_failure_is_reported(gpu):
         assert rel(b.cpu().numpy(), ref) < 1e-2
 
 
+@pytest.mark.parametrize("shapes", [[(512, 512)] * 4, [(1536, 512)], [(1536, 512), (128, 4), (37, 101)], [(700, 330)],
+                                    [(1040, 960)], [(330, 300), (20, 60)]],
+                         ids=["256-tiles", "one-large", "with-small", "tall-ragged", "272-tiles", "pinned"])
+def test_ns_default_placement_identical(gpu, shapes):
+    """The placement chosen by shape gives the device-wide queue's matrices bit for bit: batches whose widest phase has
+    up to one 64x64 tile per CU, one just past that, and one that is pinned to XCDs."""
+    mats = [rng.normal(0x370 + i, r * c, 0.0, 0.02).reshape(r, c).astype(np.float32) for i, (r, c) in enumerate(shapes)]
+    D.ns_status()
+    out = {}
+    try:
+        for mode in (0, 1):
+            D.ns_set_queues(mode)
+            out[mode] = [torch.from_numpy(m).cuda() for m in mats]
+            D.newton_schulz_batch(out[mode], coeffs=O.BASELINE_COEFFS, math="bf16")
+            D.ns_status()
+    finally:
+        D.ns_set_queues(0)
+    for a, b in zip(out[0], out[1]):
+        assert torch.equal(a, b)
+    for m, b in zip(mats, out[0]):  # the iteration in f64
+        y = torch.from_numpy(m).double().cuda()
+        y = y.t().contiguous() if m.shape[0] > m.shape[1] else y
+        y = y / (y.norm() + 1e-7)
+        for ca, cb, cc in O.BASELINE_COEFFS:
+            g = y @ y.t()
+            y = ca * y + (cb * g + cc * (g @ g)) @ y
+        y = y.t() if m.shape[0] > m.shape[1] else y
+        assert rel(b.cpu().numpy(), y.cpu().numpy()) < 1e-2
+
+
 @pytest.mark.parametrize("shape", [(1, 1), (1, 7), (3, 128), (31, 33), (32, 512), (33, 32), (64, 64), (65, 127),
                                    (96, 160), (128, 4), (128, 128), (100, 128), (160, 96), (512, 5), (129, 128),
                                    (32, 513), (97, 161)])

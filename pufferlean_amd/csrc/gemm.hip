@@ -19,6 +19,7 @@
 // second kernel adds them in split order (deterministic).
 #include "common.hpp"
 #include "kernels.hpp"
+#include "routes.hpp"
 
 #include <type_traits>
 #include <utility>
@@ -1827,7 +1828,6 @@ int gemm(const PhGemmDesc& d_in, hipStream_t st) {
   const long tiles128 = (long)((d.M + 127) / 128) * ((d.N + 127) / 128);
   const long tiles64 = (long)((d.M + 63) / 64) * ((d.N + 63) / 64);
   const bool big_ok = d.math == PH_MATH_BF16 && d.a_dtype == PH_BF16 && d.b_dtype == PH_BF16;
-  const bool f32m = d.math == PH_MATH_F32;
   bool small = false, big = big_ok && tiles256x128 >= 512, wide_n = false;
   // NT outputs at most 64 wide (the policy heads): 256x64 tiles, half the wasted columns of 256x128
   int big_bn = !d.trans_a && d.trans_b && d.N <= 64 ? 64 : 128;
@@ -1847,12 +1847,9 @@ int gemm(const PhGemmDesc& d_in, hipStream_t st) {
       // once the output has >= 16 tiles (512x512x16384: 32 -> 16 splits, 31.8 -> 26.4 us: half the
       // fp32 partials to write and fold)
       const long tw = (long)((d.M + 127) / 128);
-      // 64x64 splits of >= 256 where 128x128 tiles are mostly padding (an output at most 64 wide or tall
-      // with fp32 operands), or where 128x128 splits of >= 512 leave most CUs idle in fp32 math, whose
-      // tiles are bound by the matrix core (fp32: 128x28x32768 66 -> 13 us, 288x96x6699 74 -> 16 us; bf16 math on
-      // fp32 operands: 128x8x65536 17 -> 10 us)
-      small = !big && !wide_n && (d.a_dtype == PH_F32 || d.b_dtype == PH_F32) &&
-              ((d.M <= 64 || d.N <= 64) || (f32m && tiles128 * (d.K / 512) < 256));
+      // 64x64 splits of >= 256 where they are the faster form
+      small = !big && !wide_n &&
+              gemm_small_splits(d.math == PH_MATH_F32, d.a_dtype == PH_F32 || d.b_dtype == PH_F32, d.trans_b, d.M, d.N, d.K);
       const long want = big ? 256 / tiles256
                             : (wide_n ? 256 / tw : (small ? 256 / tiles64 : (tiles128 >= 16 ? 256 : 512) / tiles128));
       const long maxs = d.K / (big ? 2048 : (small ? 256 : 512));

@@ -1,0 +1,26 @@
+// Which form of a kernel a call takes, by sizes and types (host code, no device types). The reasons and the
+// measured times on both sides of each line stand here, at the line. All forms of one call compute the
+// same values to their tolerance, so a line's place is a matter of time only.
+#pragma once
+
+namespace ph {
+
+// ---- GEMM, reductions of k >= 4096 with a small output ------------------------------------------------
+// 64x64 split tiles instead of 128x128 ones, for outputs at most 64 wide or tall with fp32 operands (128x128 tiles
+// are mostly padding there) and, in fp32 math, where 128x128 splits of >= 512 leave most CUs idle. fp32 math is bound
+// by the matrix core, so the smaller tile wins until its tiles outnumber half the CUs and no split is left
+// (TN 128x28x32768 69 -> 17 us, 288x96x6699 89 -> 19, 512x64x262144 457 -> 317; but NT 64x8256x16384 397 -> 432).
+// With bf16 products the operand reads bound it: 64x64 tiles re-read the wide operand's partner once per tile and
+// run fewer, longer splits, so they stay to few tiles or short reductions (64x64x65536 20 -> 12 us, 128x64x262144
+// 49 -> 36, 64x1024x8192 20 -> 14.5, 64x4096x8192 38 -> 35; but 64x8256x4096 41 -> 58, 512x64x32768 23 -> 26,
+// 512x32x262144 111 -> 131).
+inline bool gemm_small_splits(bool f32_math, bool f32_operand, bool trans_b, long M, long N, long K) {
+  if (!f32_operand) return false;
+  const long tiles64 = ((M + 63) / 64) * ((N + 63) / 64), tiles128 = ((M + 127) / 128) * ((N + 127) / 128);
+  if (f32_math && tiles128 * (K / 512) < 256) return true;
+  if (M > 64 && N > 64) return false;
+  if (f32_math) return tiles64 <= 128 || !trans_b;
+  return tiles64 <= 2 || tiles64 * K <= 131072 || (tiles64 <= 64 && K <= 8192);
+}
+
+}  // namespace ph

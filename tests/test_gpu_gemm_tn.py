@@ -61,3 +61,25 @@ def test_mingru_gradient_odd_rows(D, B, T):
     err = ((G.double() - ref).norm() / ref.norm()).item()
     print(f"mingru odd rows B={B} T={T}: {err:.2e}", flush=True)
     assert err < 1e-5
+
+
+@pytest.mark.parametrize("M,N,K,ta,tb", [(64, 8256, 4096, 1, 0), (64, 8256, 4100, 0, 1), (9000, 32, 4097, 1, 0), (9000, 30, 4096, 0, 1),
+                                         (512, 64, 16384, 1, 0), (512, 64, 16392, 1, 0), (64, 130, 70001, 1, 0), (48, 100, 5003, 0, 0)])
+@pytest.mark.parametrize("math", ["f32", "bf16"])
+def test_narrow_outputs(D, M, N, K, ta, tb, math):
+    """Long reductions with an output at most 64 wide or tall, on both sides of the rule for 64x64 split tiles. The bar as
+    above; rows past the end hold NaN."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+
+    def operand(r, c):
+        x = torch.full((r + 4, c), float("nan"), device="cuda")
+        x[:r] = torch.randn(r, c, generator=g, device="cuda")
+        return x[:r]
+    a = operand(*((K, M) if ta else (M, K)))
+    b = operand(*((N, K) if tb else (K, N)))
+    out = D.gemm(a, b, trans_a=bool(ta), trans_b=bool(tb), math=math)
+    r = (lambda x: x.bfloat16().double()) if math == "bf16" else (lambda x: x.double())
+    ref = (r(a).t() if ta else r(a)) @ (r(b).t() if tb else r(b))
+    err = ((out.double() - ref).norm() / ref.norm()).item()
+    print(f"{M}x{N}x{K} ta={ta} tb={tb} {math}: {err:.2e}", flush=True)
+    assert err < 1e-5

@@ -1,0 +1,54 @@
+"""The rules that choose a kernel's form (csrc/routes.hpp) on the host, at sizes where the other form measured slower."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+DRIVER = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include "routes.hpp"
+using namespace ph;
+int main(int argc, char** argv) {
+  long a[8] = {};
+  for (int i = 2; i < argc && i < 10; i++) a[i - 2] = std::atol(argv[i]);
+  long r = -1;
+  if (!std::strcmp(argv[1], "gemm_small_splits")) r = gemm_small_splits(a[0], a[1], a[2], a[3], a[4], a[5]);
+  std::printf("%ld\n", r);
+  return 0;
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def route(tmp_path_factory):
+    d = tmp_path_factory.mktemp("routes")
+    (d / "drv.cpp").write_text(DRIVER)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Werror", "-I", os.path.join(ROOT, "pufferlean_amd", "csrc"),
+                    "-o", str(d / "drv"), str(d / "drv.cpp")], check=True)
+
+    def call(name, *args):
+        out = subprocess.run([str(d / "drv"), name] + [str(int(x)) for x in args], capture_output=True, text=True, check=True)
+        return int(out.stdout)
+    return call
+
+
+# (fp32 math, trans_b, M, N, K) of products of fp32 operands, and whether 64x64 splits are the faster form
+GEMM = [
+    (0, 0, 64, 8256, 4096, 0), (0, 0, 64, 8256, 32768, 0), (0, 1, 64, 8256, 16384, 0), (0, 0, 16, 9000, 8192, 0),
+    (0, 0, 8256, 64, 8192, 0), (0, 1, 9000, 32, 8192, 0), (0, 0, 512, 64, 32768, 0), (0, 0, 512, 32, 262144, 0),
+    (0, 0, 2048, 32, 32768, 0), (0, 0, 64, 256, 65536, 0), (0, 0, 64, 64, 65536, 1), (0, 0, 128, 64, 262144, 1),
+    (0, 0, 64, 1024, 8192, 1), (0, 0, 64, 4096, 8192, 1), (0, 1, 64, 5120, 8192, 0),
+    (0, 0, 512, 32, 8192, 1), (0, 0, 65, 65, 65536, 0), (1, 1, 64, 8256, 16384, 0),
+    (1, 1, 9000, 32, 8192, 0), (1, 0, 64, 8256, 16384, 1), (1, 1, 64, 4096, 8192, 1), (1, 0, 512, 64, 262144, 1),
+    (1, 0, 288, 96, 6699, 1), (1, 0, 512, 512, 16384, 0), (1, 0, 128, 256, 65536, 0),
+]
+
+
+@pytest.mark.parametrize("f32,tb,M,N,K,small", GEMM)
+def test_gemm_small_splits(route, f32, tb, M, N, K, small):
+    assert route("gemm_small_splits", f32, 1, tb, M, N, K) == small
+    assert route("gemm_small_splits", 0, 0, tb, M, N, K) == 0  # bf16 operands never

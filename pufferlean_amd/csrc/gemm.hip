@@ -1546,8 +1546,8 @@ __global__ void __launch_bounds__(256) k_gemm_f32(GemmArgs g) {
 
 // Split-K fold: C = epilogue(sum over splits). Bound by load latency for the small outputs that take many
 // splits (a 128x8 gradient of 128 splits: 4 blocks of one serial chain of loads each took 8 us), so ZG
-// threads share an element: each adds a contiguous range of the splits in order, sixteen loads in
-// flight, and the ranges are added in order through LDS. The order is fixed by the shape.
+// threads (fold_threads) share an element: each adds a contiguous range of the splits in order, sixteen
+// loads in flight, and the ranges are added in order through LDS. The order is fixed by the shape.
 template <typename TC, int ZG>
 __global__ void __launch_bounds__(256) k_splitk_reduce(GemmArgs g, int splits) {
   constexpr int E = 256 / ZG;  // elements per block
@@ -1578,12 +1578,12 @@ __global__ void __launch_bounds__(256) k_splitk_reduce(GemmArgs g, int splits) {
   }
   if (idx < MN) epilogue_store<TC>(g, (int)(idx / g.N), (int)(idx % g.N), s);
 }
-// Threads per element: as many as leave each >= 8 splits, while the grid stays within about 2048 blocks.
 template <typename TC>
 void launch_splitk_reduce(const GemmArgs& g, int splits, hipStream_t st) {
   const long MN = (long)g.M * g.N;
-  if (splits >= 64 && MN <= 32 * 1024) k_splitk_reduce<TC, 16><<<ceil_div(MN, 16), 256, 0, st>>>(g, splits);
-  else if (splits >= 32 && MN <= 128 * 1024) k_splitk_reduce<TC, 4><<<ceil_div(MN, 64), 256, 0, st>>>(g, splits);
+  const int zg = fold_threads(splits, MN);
+  if (zg == 16) k_splitk_reduce<TC, 16><<<ceil_div(MN, 16), 256, 0, st>>>(g, splits);
+  else if (zg == 4) k_splitk_reduce<TC, 4><<<ceil_div(MN, 64), 256, 0, st>>>(g, splits);
   else k_splitk_reduce<TC, 1><<<ceil_div(MN, 256), 256, 0, st>>>(g, splits);
 }
 

@@ -23,4 +23,14 @@ inline bool gemm_small_splits(bool f32_math, bool f32_operand, bool trans_b, lon
   return tiles64 <= 2 || tiles64 * K <= 131072 || (tiles64 <= 64 && K <= 8192);
 }
 
+// Threads per element of the split-K fold (each adds a contiguous range of the splits). One thread per element
+// has sixteen loads in flight and reads whole rows of a split; more threads shorten its chain of loads but read
+// shorter runs of a row. From 64 splits four are faster (64x64 of 128 splits 17.8 -> 14.4 us with the product, 256x256
+// of 64 31.6 -> 30.3), sixteen only for outputs of a few blocks and 256 splits (8x8x262144 19.8 -> 17.0, but 128x128 of
+// 128 splits 17.0 -> 18.3); at 16 and 32 splits one is (64x64x8192 12.7 against 13.4).
+inline int fold_threads(int splits, long MN) {
+  if (splits >= 256 && MN <= 4096) return 16;
+  return splits >= 64 && MN <= 65536 ? 4 : 1;
+}
+
 }  // namespace ph

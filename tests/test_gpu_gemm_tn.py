@@ -83,3 +83,18 @@ def test_narrow_outputs(D, M, N, K, ta, tb, math):
     err = ((out.double() - ref).norm() / ref.norm()).item()
     print(f"{M}x{N}x{K} ta={ta} tb={tb} {math}: {err:.2e}", flush=True)
     assert err < 1e-5
+
+
+@pytest.mark.parametrize("M,N,splits", [(64, 64, 63), (64, 64, 64), (64, 64, 255), (64, 64, 256), (72, 64, 256), (256, 256, 65),
+                                        (264, 256, 65), (8, 8, 300)])
+@pytest.mark.parametrize("cdt", [torch.float32, torch.bfloat16])
+def test_fold_forms(D, M, N, splits, cdt):
+    """One, four and sixteen threads per element of the fold, around the lines between them, with whole and ragged ranges
+    of splits (64 of k each, the last shorter). bf16 outputs are the rounded sums: 2^-8 per element."""
+    K = 64 * splits - 13
+    g = torch.Generator(device="cuda").manual_seed(M + splits)
+    a, b = (torch.randn(K, n, generator=g, device="cuda") for n in (M, N))
+    out = D.gemm(a, b, trans_a=True, math="f32", splits=splits, out_dtype=cdt)
+    ref = a.double().t() @ b.double()
+    err = ((out.double() - ref).norm() / ref.norm()).item()
+    assert err < (1e-5 if cdt == torch.float32 else 2 ** -8)

@@ -17,6 +17,7 @@ int main(int argc, char** argv) {
   for (int i = 2; i < argc && i < 10; i++) a[i - 2] = std::atol(argv[i]);
   long r = -1;
   if (!std::strcmp(argv[1], "gemm_small_splits")) r = gemm_small_splits(a[0], a[1], a[2], a[3], a[4], a[5]);
+  if (!std::strcmp(argv[1], "fold_threads")) r = fold_threads((int)a[0], a[1]);
   std::printf("%ld\n", r);
   return 0;
 }
@@ -52,3 +53,10 @@ GEMM = [
 def test_gemm_small_splits(route, f32, tb, M, N, K, small):
     assert route("gemm_small_splits", f32, 1, tb, M, N, K) == small
     assert route("gemm_small_splits", 0, 0, tb, M, N, K) == 0  # bf16 operands never
+
+
+@pytest.mark.parametrize("splits,MN,threads", [(128, 128 * 128, 4), (128, 64 * 512, 4), (256, 256 * 128, 4), (64, 256 * 256, 4),
+                                               (32, 64 * 64, 1), (32, 512 * 64, 1), (16, 512 * 512, 1), (64, 512 * 256, 1),
+                                               (512, 8 * 8, 16), (512, 128 * 64, 4)])
+def test_fold_threads(route, splits, MN, threads):
+    assert route("fold_threads", splits, MN) == threads

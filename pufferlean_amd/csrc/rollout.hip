@@ -18,6 +18,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "routes.hpp"
 
 // The sampler's formulas execute in the order written (no fused multiply-add), as in the CPU twin.
 #pragma clang fp contract(off)
@@ -43,8 +44,8 @@ __device__ __forceinline__ double lg(double x) { return log(x); }
 // logit type (the running sum and logp are in R; u is always f64, as in the reference's f32 form).
 // Bound by latency (one row per lane, 17 columns at a rollout): with AMAX > 0 (A <= AMAX) the row is loaded
 // into registers at once and each exponential is formed once, in blocks of one wavefront so that 4096 rows
-// spread over 64 CUs; AMAX = 0 reads wider rows from memory in each pass. The same expressions in the same
-// order: 4096 rows of 17, 8.3 -> 4.7 us.
+// spread over 64 CUs; AMAX = 0 reads the row from memory in each pass (sample_registers chooses). The same
+// expressions in the same order: 4096 rows of 16, 8.4 -> 3.8 us.
 template <typename R, bool OUT3, int AMAX>
 __global__ void __launch_bounds__(256) k_sample_cat(const R* __restrict__ Y, long ldy, long N, int A,
                                                     int has_value, unsigned long long rng, int* __restrict__ act,
@@ -411,7 +412,7 @@ PhGemmDesc nt_f32(int M, int N, int K, const float* A, long lda, const float* B,
 int sample_actions(int dtype, const void* Y, size_t ldy, size_t N, size_t A, int has_value, uint64_t rng, int* act,
                    void* logp, void* val, double* out3, hipStream_t st) {
   if (N == 0) return PH_OK;
-  // rows up to 16 or 32 logits in registers, 64 rows a block
+  // rows in registers: 64 rows a block
   auto go = [&](auto zero, auto amax) {
     using R = decltype(zero);
     constexpr int AM = decltype(amax)::value, BT = AM ? 64 : 256;
@@ -424,9 +425,13 @@ int sample_actions(int dtype, const void* Y, size_t ldy, size_t N, size_t A, int
                                                   (R*)logp, (R*)val, nullptr);
   };
   auto width = [&](auto zero) {
-    if (A <= 16) go(zero, std::integral_constant<int, 16>{});
-    else if (A <= 32) go(zero, std::integral_constant<int, 32>{});
-    else go(zero, std::integral_constant<int, 0>{});
+    switch (sample_registers((long)A)) {
+      case 4: go(zero, std::integral_constant<int, 4>{}); break;
+      case 8: go(zero, std::integral_constant<int, 8>{}); break;
+      case 16: go(zero, std::integral_constant<int, 16>{}); break;
+      case 32: go(zero, std::integral_constant<int, 32>{}); break;
+      default: go(zero, std::integral_constant<int, 0>{});
+    }
   };
   if (dtype == PH_F64) width(0.0);
   else width(0.f);

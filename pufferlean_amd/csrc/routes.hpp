@@ -33,4 +33,14 @@ inline int fold_threads(int splits, long MN) {
   return splits >= 64 && MN <= 65536 ? 4 : 1;
 }
 
+// ---- Categorical sampler ----------------------------------------------------------------------------------
+// Logits of a row held in registers (4, 8, 16 or 32; every one is loaded and exponentiated, so the least that holds
+// the row), or 0: the row is read from memory in each pass. That form stays for one action and past 32.
+// fp32, 4 actions: 4096 rows 3.7 us in passes, 3.1 in 16 registers, 2.4 in 4; 1048576 rows 12.7, 15.2 and 8.3
+// (one action 7.0, 13.4 and 7.6).
+inline int sample_registers(long A) {
+  if (A <= 1 || A > 32) return 0;
+  return A <= 4 ? 4 : A <= 8 ? 8 : A <= 16 ? 16 : 32;
+}
+
 }  // namespace ph

@@ -65,9 +65,9 @@ def test_step(D, N, H, A, L, precision):
 
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.float64])
-@pytest.mark.parametrize("A", [1, 2, 15, 16, 17, 32, 33])
+@pytest.mark.parametrize("A", [1, 2, 4, 5, 8, 9, 15, 16, 17, 32, 33])
 def test_sampler_widths(D, A, dt):
-    """Register forms (up to 16 and 32 logits) and the wide form against numpy's softmax and inverse CDF; a draw
+    """Register forms (up to 4, 8, 16 and 32 logits) and the wide form against numpy's softmax and inverse CDF; a draw
     within 1e-5 (f32) or 1e-12 (f64) of a cumulative boundary may take the neighbour."""
     from pufferlean_amd import rng
     N = 777

@@ -18,6 +18,7 @@ int main(int argc, char** argv) {
   long r = -1;
   if (!std::strcmp(argv[1], "gemm_small_splits")) r = gemm_small_splits(a[0], a[1], a[2], a[3], a[4], a[5]);
   if (!std::strcmp(argv[1], "fold_threads")) r = fold_threads((int)a[0], a[1]);
+  if (!std::strcmp(argv[1], "sample_registers")) r = sample_registers(a[0]);
   std::printf("%ld\n", r);
   return 0;
 }
@@ -60,3 +61,8 @@ def test_gemm_small_splits(route, f32, tb, M, N, K, small):
                                                (512, 8 * 8, 16), (512, 128 * 64, 4)])
 def test_fold_threads(route, splits, MN, threads):
     assert route("fold_threads", splits, MN) == threads
+
+
+@pytest.mark.parametrize("A,regs", [(1, 0), (2, 4), (4, 4), (5, 8), (8, 8), (9, 16), (16, 16), (17, 32), (32, 32), (33, 0)])
+def test_sample_registers(route, A, regs):
+    assert route("sample_registers", A) == regs

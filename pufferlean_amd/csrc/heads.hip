@@ -8,6 +8,7 @@
 // One lane per row, as the heads are a few dozen columns wide; each row's head outputs are read once
 // and its gradient row written once.
 #include <cmath>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -104,21 +105,46 @@ __global__ void __launch_bounds__(256) k_ppo_grad_md(const float* __restrict__ o
 // are skipped) and the gradient rows leave through the same tile. The pitch is odd (O, or O + 1 for even
 // rows), so the lanes reading one column of their rows hit distinct banks; where it equals both the row width
 // and the stride, the block's rows are one run of floats and move with 16-byte loads and stores. Each lane works on
-// its row in LDS, so a block holds only its rows (250007x15: 19 KB) and eight are resident per CU, whose load,
-// compute and store phases overlap: 977 blocks are one round of the chip. Loops over a head's columns are
-// unrolled with an exit at the head's size, which is the same for every lane.
-// 250007 rows, heads 9 and 5, with losses: 27.0 -> 17.0 us (a tile of 33-float rows with the row and the
-// probabilities in 32 masked registers each, four blocks per CU).
+// its row in LDS, so a block holds only its rows (250007x15: 19 KB); registers bound the blocks per CU (four or
+// five), whose load, compute and store phases overlap. Loops over a head's columns are unrolled with an exit at
+// the head's size, which is the same for every lane; heads past 12 columns take one pass of 16 or 32 masked ones,
+// whose exponentials run side by side (one head of 31, 4096 rows: 24.6 us with exits, 16.3 masked; heads of 9 and 5
+// at 250007 rows 27.0 masked, 20 with exits). 4096 rows at a stride of 32: heads 9 and 5 15.4 -> 12.8 us.
 constexpr int kTileW = 32;
 constexpr int kRows = 256;
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 // Lane t walks the (row, column) pairs t, t + 256, ... of the R x O block in row-major order; the
-// pair advances by 256 / O rows and 256 % O columns with a carry, so no division runs per element.
+// pair advances by 256 / O rows and 256 % O columns with a carry, so no division runs per element. A lane's
+// share is at most O <= NI elements; every load is issued before the first LDS store waits on one, with no exit
+// among them (a branch between loads makes them wait for one another).
+template <int NI>
+__device__ __forceinline__ void tile_pull(const float* __restrict__ s, long ld, int O, int P, int R,
+                                          float* __restrict__ tile) {
+  const int t = threadIdx.x, q = kRows / O, rm = kRows % O;
+  int r = t / O, c = t % O;
+  float v[NI];
+  int dst[NI];
+#pragma unroll
+  for (int it = 0; it < NI; it++) {
+    dst[it] = -1;
+    if (r < R) {
+      v[it] = s[(long)r * ld + c];
+      dst[it] = r * P + c;
+    }
+    r += q;
+    c += rm;
+    if (c >= O) {
+      c -= O;
+      r++;
+    }
+  }
+#pragma unroll
+  for (int it = 0; it < NI; it++)
+    if (dst[it] >= 0) tile[dst[it]] = v[it];
+}
 __device__ __forceinline__ void tile_load(const float* __restrict__ src, long ld, int O, int P, long n0, int R,
                                           bool linear, float* __restrict__ tile) {
-  // a lane's share is at most kTileW elements (R * O <= 256 * kTileW): every load is issued before
-  // the first LDS store waits on one
   const int t = threadIdx.x, tot = R * O;
   const float* s = src + n0 * ld;
   if (linear) {
@@ -138,30 +164,9 @@ __device__ __forceinline__ void tile_load(const float* __restrict__ src, long ld
     }
     return;
   }
-  const int q = kRows / O, rm = kRows % O;
-  int r = t / O, c = t % O;
-  float v[kTileW];
-  int dst[kTileW];
-#pragma unroll
-  for (int it = 0; it < kTileW; it++) {
-    if (it * kRows >= tot) break;
-    dst[it] = -1;
-    if (r < R) {
-      v[it] = s[(long)r * ld + c];
-      dst[it] = r * P + c;
-    }
-    r += q;
-    c += rm;
-    if (c >= O) {
-      c -= O;
-      r++;
-    }
-  }
-#pragma unroll
-  for (int it = 0; it < kTileW; it++) {
-    if (it * kRows >= tot) break;
-    if (dst[it] >= 0) tile[dst[it]] = v[it];
-  }
+  if (O <= 8) tile_pull<8>(s, ld, O, P, R, tile);
+  else if (O <= 16) tile_pull<16>(s, ld, O, P, R, tile);
+  else tile_pull<kTileW>(s, ld, O, P, R, tile);
 }
 __device__ __forceinline__ void tile_store(float* __restrict__ dst, long ld, int O, int P, long n0, int R, bool linear,
                                            const float* __restrict__ tile) {
@@ -196,6 +201,8 @@ static bool linear_rows(const float* p, size_t ld, int O) { return ld == (size_t
 constexpr int kTileHeads = 8;
 static size_t md_tile_lds(int O, size_t K) { return (size_t)kRows * ((O | 1) + 2 * K) * 4; }
 static_assert((size_t)kRows * ((kTileW | 1) + 2 * kTileHeads) * 4 <= kMaxLdsBytes, "LDS budget");
+// HW > 0: the columns of a head run in one pass of HW masked ones (HW at least every head's size); 0: with exits.
+template <int HW>
 __global__ void __launch_bounds__(kRows) k_ppo_grad_md_tile(const float* __restrict__ out, long ldo,
                                                             const int* __restrict__ act, const float* __restrict__ adv,
                                                             const float* __restrict__ ret, const float* __restrict__ old,
@@ -241,18 +248,29 @@ __global__ void __launch_bounds__(kRows) k_ppo_grad_md_tile(const float* __restr
     for (int h = 0; h < K; h++) {
       const int sz = hs.n[h], ah = acts[h * kRows + t];
       float x[kTileW];
-      float m = -INFINITY;
+      float m = -INFINITY, se = 0.f;
+      if constexpr (HW > 0) {
 #pragma unroll
-      for (int k = 0; k < kTileW; k++) {
-        if (k >= sz) break;
-        x[k] = row[off + k];
-        m = fmaxf(m, x[k]);
-      }
-      float se = 0.f;
+        for (int k = 0; k < HW; k++) x[k] = row[off + min(k, sz - 1)];
 #pragma unroll
-      for (int k = 0; k < kTileW; k++) {
-        if (k >= sz) break;
-        se += expf(x[k] - m);
+        for (int k = 0; k < HW; k++) m = fmaxf(m, x[k]);
+#pragma unroll
+        for (int k = 0; k < HW; k++) x[k] = expf(x[k] - m);
+#pragma unroll
+        for (int k = 0; k < HW; k++)
+          if (k < sz) se += x[k];
+      } else {
+#pragma unroll
+        for (int k = 0; k < kTileW; k++) {
+          if (k >= sz) break;
+          x[k] = row[off + k];
+          m = fmaxf(m, x[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < kTileW; k++) {
+          if (k >= sz) break;
+          se += expf(x[k] - m);
+        }
       }
       const float lse = m + logf(se);
       lses[h * kRows + t] = lse;
@@ -271,22 +289,38 @@ __global__ void __launch_bounds__(kRows) k_ppo_grad_md_tile(const float* __restr
       const float lse = lses[h * kRows + t];
       float x[kTileW], p[kTileW];
       float po = 0.f;
+      if constexpr (HW > 0) {
 #pragma unroll
-      for (int k = 0; k < kTileW; k++) {
-        if (k >= sz) break;
-        x[k] = row[off + k];
-      }
+        for (int k = 0; k < HW; k++) x[k] = row[off + min(k, sz - 1)];
 #pragma unroll
-      for (int k = 0; k < kTileW; k++) {
-        if (k >= sz) break;
-        p[k] = expf(x[k] - lse);
-        po += p[k] * x[k];
-        entropy -= p[k] * (x[k] - lse);
-      }
+        for (int k = 0; k < HW; k++) p[k] = expf(x[k] - lse);
 #pragma unroll
-      for (int k = 0; k < kTileW; k++) {
-        if (k >= sz) break;
-        row[off + k] = dPol * ((k == ah ? 1.f : 0.f) - p[k]) + ent * p[k] * (po - x[k]);
+        for (int k = 0; k < HW; k++)
+          if (k < sz) {
+            po += p[k] * x[k];
+            entropy -= p[k] * (x[k] - lse);
+          }
+#pragma unroll
+        for (int k = 0; k < HW; k++)
+          if (k < sz) row[off + k] = dPol * ((k == ah ? 1.f : 0.f) - p[k]) + ent * p[k] * (po - x[k]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < kTileW; k++) {
+          if (k >= sz) break;
+          x[k] = row[off + k];
+        }
+#pragma unroll
+        for (int k = 0; k < kTileW; k++) {
+          if (k >= sz) break;
+          p[k] = expf(x[k] - lse);
+          po += p[k] * x[k];
+          entropy -= p[k] * (x[k] - lse);
+        }
+#pragma unroll
+        for (int k = 0; k < kTileW; k++) {
+          if (k >= sz) break;
+          row[off + k] = dPol * ((k == ah ? 1.f : 0.f) - p[k]) + ent * p[k] * (po - x[k]);
+        }
       }
       off += sz;
     }
@@ -302,6 +336,9 @@ __global__ void __launch_bounds__(kRows) k_ppo_grad_md_tile(const float* __restr
 }
 
 // k_ppo_grad_cont for 2d + 1 <= kTileW.
+// MASK: every loop over dimensions runs all of them, masked (strided rows of more than four: 262144 rows of 15
+// dimensions 43.7 us with exits here and in the load, 28.1 masked; packed rows 28.7 with exits).
+template <bool MASK>
 __global__ void __launch_bounds__(kRows) k_ppo_grad_cont_tile(const float* __restrict__ out, long ldo,
                                                               const float* __restrict__ act, const float* __restrict__ adv,
                                                               const float* __restrict__ ret, const float* __restrict__ old,
@@ -322,8 +359,8 @@ __global__ void __launch_bounds__(kRows) k_ppo_grad_cont_tile(const float* __res
   if (t < R) {
 #pragma unroll
     for (int i = 0; i < DM; i++) {
-      if (i >= d) break;
-      av[i] = act[n * d + i];
+      if (!MASK && i >= d) break;
+      av[i] = act[n * d + (MASK ? min(i, d - 1) : i)];
     }
     A = adv[n];
     rv = ret[n];
@@ -335,29 +372,46 @@ __global__ void __launch_bounds__(kRows) k_ppo_grad_cont_tile(const float* __res
   double lsum[6] = {0, 0, 0, 0, 0, 0};
   if (t < R) {
     float* row = tile + t * P;
-    float z[DM];
+    float z[DM], lsr[DM];
     const float vnew = row[W];
     const float hl = (float)kHalfLog2Pi;
     float logp = 0.f, entropy = 0.f;
+    if constexpr (MASK) {
+      float mu[DM];
+#pragma unroll
+      for (int i = 0; i < DM; i++) {
+        mu[i] = row[min(i, d - 1)];
+        lsr[i] = row[d + min(i, d - 1)];
+      }
+#pragma unroll
+      for (int i = 0; i < DM; i++) z[i] = av[i] - mu[i];
+    }
 #pragma unroll
     for (int i = 0; i < DM; i++) {
-      if (i >= d) break;
-      const float lsr = row[d + i];
-      const float ls = lsr < lslo ? lslo : (lsr > lshi ? lshi : lsr);
-      z[i] = (av[i] - row[i]) * expf(-ls);
-      logp += -0.5f * z[i] * z[i] - ls - hl;
-      entropy += ls + (0.5f + hl);
+      if (!MASK && i >= d) break;
+      if (!MASK) {
+        lsr[i] = row[d + i];
+        z[i] = av[i] - row[i];
+      }
+      const float ls = lsr[i] < lslo ? lslo : (lsr[i] > lshi ? lshi : lsr[i]);
+      z[i] = z[i] * expf(-ls);
+      if (!MASK || i < d) {
+        logp += -0.5f * z[i] * z[i] - ls - hl;
+        entropy += ls + (0.5f + hl);
+      }
     }
     const float ratio = expf(logp - ol), lo = 1.f - clip, hi = 1.f + clip;
     const float rc = ratio < lo ? lo : (ratio > hi ? hi : ratio);
     const float dPol = (A * ratio <= A * rc) ? A * ratio : ((lo < ratio && ratio < hi) ? A * ratio : 0.f);
 #pragma unroll
     for (int i = 0; i < DM; i++) {
-      if (i >= d) break;
-      const float lsr = row[d + i];
-      const float ls = lsr < lslo ? lslo : (lsr > lshi ? lshi : lsr);
-      row[i] = dPol * z[i] * expf(-ls);
-      row[d + i] = (lslo < lsr && lsr < lshi) ? dPol * (z[i] * z[i] - 1.f) + ent : 0.f;
+      if (!MASK && i >= d) break;
+      const float ls = lsr[i] < lslo ? lslo : (lsr[i] > lshi ? lshi : lsr[i]);
+      const float g = dPol * z[i] * expf(-ls);
+      if (!MASK || i < d) {
+        row[i] = g;
+        row[d + i] = (lslo < lsr[i] && lsr[i] < lshi) ? dPol * (z[i] * z[i] - 1.f) + ent : 0.f;
+      }
     }
     row[W] = -vf * vloss_grad(vnew, rv, vold, ov != nullptr, vfClip);
     if (newlp) newlp[n] = logp;
@@ -518,11 +572,18 @@ int ppo_grad_md(const float* out, size_t ldo, const int* act, const float* adv, 
   const unsigned grid = ceil_div(N, 256);
   double* part;
   PH_TRY(loss_part(losses, grid, part));
-  if (W + 1 <= kTileW && K <= (size_t)kTileHeads)
-    k_ppo_grad_md_tile<<<grid, kRows, md_tile_lds(W + 1, K), st>>>(
-        out, (long)ldo, act, adv, ret, old, ov, (long)N, hs, W, vf, ent, clip, vfClip, dout, (long)ldd,
-        linear_rows(out, ldo, W + 1), linear_rows(dout, ldd, W + 1), newlp, newval, part, losses);
-  else
+  if (W + 1 <= kTileW && K <= (size_t)kTileHeads) {
+    int widest = 0;
+    for (size_t h = 0; h < K; h++) widest = hs.n[h] > widest ? hs.n[h] : widest;
+    auto go = [&](auto hw) {
+      k_ppo_grad_md_tile<decltype(hw)::value><<<grid, kRows, md_tile_lds(W + 1, K), st>>>(
+          out, (long)ldo, act, adv, ret, old, ov, (long)N, hs, W, vf, ent, clip, vfClip, dout, (long)ldd,
+          linear_rows(out, ldo, W + 1), linear_rows(dout, ldd, W + 1), newlp, newval, part, losses);
+    };
+    if (widest > 16) go(std::integral_constant<int, 32>{});
+    else if (widest > 12) go(std::integral_constant<int, 16>{});
+    else go(std::integral_constant<int, 0>{});
+  } else
     k_ppo_grad_md<<<grid, 256, 0, st>>>(out, (long)ldo, act, adv, ret, old, ov, (long)N, hs, W, vf, ent, clip, vfClip,
                                         dout, (long)ldd, newlp, newval, part, losses);
   PH_LAUNCH_CHECK();
@@ -538,11 +599,16 @@ int ppo_grad_cont(const float* out, size_t ldo, const float* act, const float* a
   const unsigned grid = ceil_div(N, 256);
   double* part;
   PH_TRY(loss_part(losses, grid, part));
-  if (2 * d + 1 <= (size_t)kTileW)
-    k_ppo_grad_cont_tile<<<grid, kRows, (size_t)kRows * (2 * d + 1) * 4, st>>>(
-        out, (long)ldo, act, adv, ret, old, ov, (long)N, (int)d, vf, ent, clip, vfClip, lslo, lshi, dout, (long)ldd,
-        linear_rows(out, ldo, 2 * (int)d + 1), linear_rows(dout, ldd, 2 * (int)d + 1), newlp, newval, part, losses);
-  else
+  if (2 * d + 1 <= (size_t)kTileW) {
+    const bool lin = linear_rows(out, ldo, 2 * (int)d + 1), linOut = linear_rows(dout, ldd, 2 * (int)d + 1);
+    auto go = [&](auto mask) {
+      k_ppo_grad_cont_tile<decltype(mask)::value><<<grid, kRows, (size_t)kRows * (2 * d + 1) * 4, st>>>(
+          out, (long)ldo, act, adv, ret, old, ov, (long)N, (int)d, vf, ent, clip, vfClip, lslo, lshi, dout, (long)ldd, lin,
+          linOut, newlp, newval, part, losses);
+    };
+    if (!lin && d > 4) go(std::true_type{});
+    else go(std::false_type{});
+  } else
     k_ppo_grad_cont<<<grid, 256, 0, st>>>(out, (long)ldo, act, adv, ret, old, ov, (long)N, (int)d, vf, ent, clip,
                                           vfClip, lslo, lshi, dout, (long)ldd, newlp, newval, part, losses);
   PH_LAUNCH_CHECK();

@@ -1,5 +1,6 @@
 """Head gradients through the LDS tile: row counts around a block's 256 rows, odd and even row widths, one to eight
-heads, packed rows (moved as one run of floats), strided rows and rows off the 16-byte alignment."""
+heads, the largest around the lines between the column passes, packed rows (moved as one run of floats), strided
+rows and rows off the 16-byte alignment."""
 import numpy as np
 import pytest
 import torch
@@ -35,7 +36,8 @@ LAYOUTS = ["packed", "strided", "offset"]
 
 
 @pytest.mark.parametrize("N", [1, 63, 255, 256, 257, 1001])
-@pytest.mark.parametrize("sizes", [[1], [2], [9, 5], [3, 3, 4, 1], [31], [1, 2, 3, 4, 5, 6, 7, 3], [12, 7, 3]])
+@pytest.mark.parametrize("sizes", [[1], [2], [9, 5], [3, 3, 4, 1], [31], [1, 2, 3, 4, 5, 6, 7, 3], [12, 7, 3],
+                                   [13, 2], [16, 15], [17, 1]])
 def test_md_tile(gpu, N, sizes):
     K, W = len(sizes), sum(sizes)
     out = f32(rng.normal(0xB01 + N, N * (W + 1)).reshape(N, W + 1) * 2.0)
@@ -63,7 +65,7 @@ def test_md_tile(gpu, N, sizes):
 
 
 @pytest.mark.parametrize("N", [1, 256, 257, 1001])
-@pytest.mark.parametrize("dim", [1, 2, 8, 15])
+@pytest.mark.parametrize("dim", [1, 2, 4, 5, 8, 15])
 def test_cont_tile(gpu, N, dim):
     w = 2 * dim + 1
     out = rng.normal(0xB11 + N, N * w).reshape(N, w)

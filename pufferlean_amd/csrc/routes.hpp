@@ -43,4 +43,23 @@ inline int sample_registers(long A) {
   return A <= 4 ? 4 : A <= 8 ? 8 : A <= 16 ? 16 : 32;
 }
 
+// ---- V-trace scan ----------------------------------------------------------------------------------------
+// Whether a batch takes the tiles of 16 or 64 segments x chunks of 64 steps staged through LDS, or one lane (two for
+// the largest fp32 batches) per segment walking its steps.
+// Time-major: from 32768 segments (f64 past 24576) the lanes alone fill the chip and stream whole rows (fp32 65536x64
+// 18.6 us against 26.1 tiled). Below that a lane is one chain of dependent load rounds that grows with T, and a
+// chunk costs the same whether its 64 steps are real or not: short horizons stay with the lanes (fp32 4096 segments,
+// lanes / tiles: T = 4 3.0 / 3.2 us, 8 3.4 / 3.3, 64 13.1 / 6.1; 16384, tiles of 64 segments: 16 5.0 / 5.7, 32 8.0 /
+// 6.6; f64 4096: 8 4.2 / 3.8, 8192: 8 4.3 / 4.5, 16384: 12 5.8 / 6.0), and where the two are close a chunk that is
+// mostly padding decides (fp32 32767 segments: 64 16.0 / 12.6, 72 16.9 / 17.6, 96 21.5 / 19.5).
+// Segment-major: lanes read T elements apart, so tiles win sooner (fp32 4096: 2 3.5 / 3.2, 4 5.3 / 3.3; 16384: 4 5.3 /
+// 6.0, 8 9.9 / 6.1; 65536: 8 10.8 / 12.1, 12 15.4 / 12.7; f64 256: 4 3.0 / 3.7, 8 5.9 / 3.8; 32767: 8 8.4 / 9.6).
+inline bool vtrace_tiled(bool f64, bool time_major, long B, long T) {
+  if (!time_major) return T >= (f64 ? (B <= 16384 ? 8 : 12) : (B <= 8192 ? 4 : B <= 32768 ? 8 : 12));
+  const long pad = (T + 63) / 64 * 64 - T;
+  if (B <= 8192) return T >= (f64 ? 12 : 8);
+  if (f64) return B <= 16384 ? T >= 16 : B <= 24576 && 2 * pad <= T;
+  return B <= 24576 ? T >= 32 : B < 32768 && 2 * pad <= T;
+}
+
 }  // namespace ph

@@ -1,16 +1,17 @@
 // V-trace / GAE reverse scan (bandwidth-bound: no MFMA).
 //
-// Large time-major batches ([T][B]): one lane per segment (two for the largest fp32 ones) walks t
-// backwards, the recurrence in registers with the done mask applied there. Loads are issued a chunk of CH
-// steps ahead of the dependent arithmetic so a lane keeps 4*CH loads in flight; consecutive segments on
-// consecutive lanes make every load and store a fully coalesced row per wavefront. Smaller batches and
-// segment-major rows ([B][T]): tiles of segments x steps staged through LDS (k_vtrace_tile).
+// Two forms, chosen by vtrace_tiled. Lanes: one lane per segment (two for the largest fp32 time-major batches)
+// walks t backwards, the recurrence in registers with the done mask applied there. Loads are issued a chunk of CH
+// steps ahead of the dependent arithmetic so a lane keeps 4*CH loads in flight; in time-major rows ([T][B])
+// consecutive segments on consecutive lanes make every load and store a fully coalesced row per wavefront. Tiles:
+// blocks of segments x steps staged through LDS (k_vtrace_tile), for smaller batches and segment-major rows ([B][T]).
 //
 // Arithmetic follows the reference's sequential op order with contraction disabled, so the f64
 // kernel is bit-identical to the reference CPU scans (puffercuda.cu:120-132, 200-211) and the f32
 // kernel is bit-identical to an f32 evaluation of the same expressions.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "routes.hpp"
 
 namespace ph {
 namespace {
@@ -62,16 +63,19 @@ __device__ __forceinline__ void stl(R* p, const Lanes<R, V>& o) {
 // VARIANT 1: bootstrapped form (delta = rho*r + g*V'*nnt - V, V' at T-1 = boot, done := term > .5).
 // rho == nullptr means ratio 1 (plain GAE). Each lane runs the recurrence of V segments side by
 // side, each in the reference's op order.
-template <typename R, int VARIANT, int CH, int V, bool NT>
+template <typename R, int VARIANT, bool TIME_MAJOR, int CH, int V, bool NT>
 __global__ void __launch_bounds__(256) k_vtrace(const R* __restrict__ rew, const R* __restrict__ val,
                                                 const R* __restrict__ term, const R* __restrict__ rho,
                                                 const R* __restrict__ boot, R* __restrict__ adv,
                                                 R* __restrict__ tgt, int B, int T, int rho_is_log,
                                                 int clamp, R gamma, R lam, R rhoClip, R cClip) {
 #pragma clang fp contract(off)
+  static_assert(V == 1 || TIME_MAJOR, "vector lanes run along b (time-major rows)");
   const int b = (blockIdx.x * blockDim.x + threadIdx.x) * V;
   if (b >= B) return;
-  auto at = [&](int t) -> size_t { return (size_t)t * (size_t)B + (size_t)b; };
+  auto at = [&](int t) -> size_t {
+    return TIME_MAJOR ? (size_t)t * (size_t)B + (size_t)b : (size_t)b * (size_t)T + (size_t)t;
+  };
   typedef Lanes<R, V> P;
   const R gl = gamma * lam;
   R last[V], vnext[V];
@@ -179,15 +183,15 @@ __device__ __forceinline__ void lds_sync() {
 }
 
 // Tiled form for batches that do not fill the chip with one lane per segment (a rollout's 4096 segments
-// are 64 wavefronts on 256 CUs, each a chain of dependent load rounds: 13.6 us for 6.3 MB), and for
-// segment-major rows, which lanes would read T elements apart. A block takes SB segments; all 256 threads
-// load a chunk of kTc steps at once, form each step's delta, clipped c and not-done factor in parallel (the
-// ratios' exponentials included), and leave them in LDS; SB lanes then run the recurrence out of LDS, one
-// multiply-multiply-add chain per segment, and all threads write the chunk. The next chunk's loads are in
-// flight during the chain. Same expressions in the same order per element as k_vtrace, so bit-identical.
-// 16 segments a block spread 4096 segments over every CU; neighbouring blocks share cache lines of a
-// time-major row, so each XCD takes a contiguous range of segments. 4096x64: fp32 time-major 12.9 -> 5.7 us,
-// segment-major 60 -> 4.9 (f64 58 -> 6.8); 4096x256 fp32 time-major 46 -> 17.7.
+// are 64 wavefronts on 256 CUs, each a chain of dependent load rounds), and for segment-major rows, which lanes
+// would read T elements apart. A block takes SB segments; all 256 threads load a chunk of kTc steps at once, form
+// each step's delta, clipped c and not-done factor in parallel (the ratios' exponentials included), and leave
+// them in LDS; SB lanes then run the recurrence out of LDS, one multiply-multiply-add chain per segment, and all
+// threads write the chunk. The next chunk's loads are in flight during the chain. Same expressions in the same
+// order per element as k_vtrace, so bit-identical. 16 segments a block spread 4096 segments over every CU;
+// neighbouring blocks share cache lines of a time-major row, so each XCD takes a contiguous range of segments.
+// 4096x64, lanes -> tiles, replayed from a graph: fp32 time-major 13.1 -> 6.1 us, segment-major 60.6 -> 5.2 (f64
+// 18.8 -> 7.0 and 58.5 -> 6.9); 4096x256 fp32 time-major 46.5 -> 17.8.
 constexpr int kTc = 64;
 template <typename R, int VARIANT, bool TIME_MAJOR, int SB>
 __global__ void __launch_bounds__(256) k_vtrace_tile(const R* __restrict__ rew, const R* __restrict__ val,
@@ -298,28 +302,29 @@ int launch_vtrace(const R* rew, const R* val, const R* term, const R* rho, const
   const bool wide = sizeof(R) == 4 && time_major && B % 2 == 0 && B >= 2 * 256 * 256 &&
                     aligned8(rew) && aligned8(val) && aligned8(term) && aligned8(rho) &&
                     aligned8(boot) && aligned8(adv) && aligned8(tgt);
-#define PH_VT(VAR, VV, NT)                                                                         \
-  k_vtrace<R, VAR, CH, VV, NT><<<ceil_div(B / VV, 256), 256, 0, st>>>(                           \
+#define PH_VT(VAR, TM, VV, NT)                                                                     \
+  k_vtrace<R, VAR, TM, CH, VV, NT><<<ceil_div(B / VV, 256), 256, 0, st>>>(                           \
       rew, val, term, rho, boot, adv, tgt, (int)B, (int)T, rho_is_log, clamp, (R)gamma, (R)lam,     \
       (R)rhoClip, (R)cClip)
   if constexpr (sizeof(R) == 4) {
     if (wide) {
-      if (variant == 0) PH_VT(0, 2, true);
-      else PH_VT(1, 2, true);
+      if (variant == 0) PH_VT(0, true, 2, true);
+      else PH_VT(1, true, 2, true);
       PH_LAUNCH_CHECK();
       return PH_OK;
     }
   }
-  // Time-major batches of 32768 segments and more fill the chip with one lane per segment (512 wavefronts),
-  // which streams whole rows: 65536x64 fp32 18.6 us against 26.1 tiled (f64 32 / 38), 16384x64 13.7 against
-  // 8.2 (f64 21 / 12). Segment-major rows are always tiled (lanes read T elements apart: 65536x64 213 / 25 us).
-  // Tiles of 16 segments while that gives at most two rounds of blocks per CU, and in f64 (64 would pass the
-  // LDS budget); 64 beyond.
-  if (time_major && B >= 32768) {
-    if (variant == 0) PH_VT(0, 1, false); else PH_VT(1, 1, false);
+  if (!vtrace_tiled(sizeof(R) == 8, time_major, (long)B, (long)T)) {
+    if (variant == 0) {
+      if (time_major) PH_VT(0, true, 1, false); else PH_VT(0, false, 1, false);
+    } else {
+      if (time_major) PH_VT(1, true, 1, false); else PH_VT(1, false, 1, false);
+    }
     PH_LAUNCH_CHECK();
     return PH_OK;
   }
+  // Tiles of 16 segments while that gives at most two rounds of blocks per CU, and in f64 (64 would pass the
+  // LDS budget); 64 beyond.
 #define PH_VTT(VAR, TM, SB)                                                                                \
   k_vtrace_tile<R, VAR, TM, SB><<<ceil_div(B, SB), 256, 0, st>>>(rew, val, term, rho, boot, adv, tgt, (int)B, \
                                                                  (int)T, rho_is_log, clamp, (R)gamma, (R)lam, \

@@ -164,7 +164,8 @@ def test_full_size_replicated_properties(gpu):
 @pytest.mark.parametrize("time_major", [True, False])
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
 @pytest.mark.parametrize("B,T", [(15, 1), (16, 63), (17, 64), (33, 65), (64, 129), (8192, 3), (8193, 5), (8257, 66),
-                                 (32767, 9), (32768, 9)])
+                                 (32767, 9), (32768, 9), (300, 7), (300, 11), (300, 12), (8193, 31), (8193, 33), (16385, 48),
+                                 (24577, 64), (32769, 12)])
 def test_tiled_scan_bit_exact(gpu, dt, B, T, time_major, variant):
     """Edges of the tiled scan (16 or 64 segments x chunks of 64 steps) and of the rule that chooses it:
     bit-identical to the sequential twin in the same precision, terminals on chunk boundaries included."""

@@ -19,6 +19,7 @@ int main(int argc, char** argv) {
   if (!std::strcmp(argv[1], "gemm_small_splits")) r = gemm_small_splits(a[0], a[1], a[2], a[3], a[4], a[5]);
   if (!std::strcmp(argv[1], "fold_threads")) r = fold_threads((int)a[0], a[1]);
   if (!std::strcmp(argv[1], "sample_registers")) r = sample_registers(a[0]);
+  if (!std::strcmp(argv[1], "vtrace_tiled")) r = vtrace_tiled(a[0], a[1], a[2], a[3]);
   std::printf("%ld\n", r);
   return 0;
 }
@@ -66,3 +67,18 @@ def test_fold_threads(route, splits, MN, threads):
 @pytest.mark.parametrize("A,regs", [(1, 0), (2, 4), (4, 4), (5, 8), (8, 8), (9, 16), (16, 16), (17, 32), (32, 32), (33, 0)])
 def test_sample_registers(route, A, regs):
     assert route("sample_registers", A) == regs
+
+
+# (f64, time-major, B, T) and whether the tiles are the faster form
+VTRACE = [(0, 1, 4096, 1, 0), (0, 1, 4096, 4, 0), (0, 1, 4096, 8, 1), (0, 1, 16384, 8, 0), (0, 1, 16384, 16, 0),
+          (0, 1, 16384, 64, 1), (0, 1, 32767, 8, 0), (0, 1, 32767, 64, 1), (0, 1, 32767, 72, 0), (0, 1, 32768, 64, 0),
+          (1, 1, 4096, 4, 0), (1, 1, 8192, 8, 0), (1, 1, 4096, 64, 1), (1, 1, 16384, 12, 0), (1, 1, 16384, 64, 1),
+          (1, 1, 24576, 16, 0), (1, 1, 24576, 65, 0), (1, 1, 24576, 128, 1), (1, 1, 32767, 65, 0), (0, 0, 4096, 1, 0),
+          (0, 0, 4096, 4, 1), (0, 0, 16384, 4, 0), (0, 0, 16384, 8, 1), (0, 0, 65536, 1, 0), (0, 0, 65536, 8, 0),
+          (0, 0, 65536, 64, 1), (1, 0, 256, 4, 0), (1, 0, 4096, 8, 1), (1, 0, 32767, 8, 0), (1, 0, 65536, 2, 0),
+          (1, 0, 65536, 64, 1)]
+
+
+@pytest.mark.parametrize("f64,tm,B,T,tiled", VTRACE)
+def test_vtrace_tiled(route, f64, tm, B, T, tiled):
+    assert route("vtrace_tiled", f64, tm, B, T) == tiled

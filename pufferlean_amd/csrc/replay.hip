@@ -26,6 +26,7 @@
 
 #include "common.hpp"
 #include "kernels.hpp"
+#include "routes.hpp"
 
 // The formulas below execute in the order written (no fused multiply-add), as in the CPU twins.
 #pragma clang fp contract(off)
@@ -42,17 +43,12 @@ constexpr int kGaBlock = kGaThreads * kGaPer;
 constexpr unsigned kFoldMax = 2048;  // gather blocks whose partials every normalising block merges itself
 constexpr int kSm = 16, kSt = 64;    // tile of segment-major columns: segments x steps
 constexpr int kSp = kSt + 1;         // its LDS pitch (a step of 16 segments hits distinct banks)
-// Segment-major columns of at least kSmMinT steps take the tiles: shorter rows fill too little of a 64-step run, and
-// their whole row is a cache line or less for the thread-per-element forms.
-constexpr int kSmMinT = 16;
-inline bool sm_tiles(const ph_replay_cols& c) {  // (the upper bound keeps a tile's steps within int)
-  return !c.time_major && c.T >= (size_t)kSmMinT && c.T <= (size_t)1 << 30;
-}
+inline bool sm_tiles(const ph_replay_cols& c) { return gather_tiled(c.time_major, (long)c.T); }
 constexpr long kScanDraws = 8192;    // draws compared pairwise by the segment-major iterate
 
 // ---- per-segment |adv| sums ------------------------------------------------------------------------
 // t ascending, f64 accumulation (the reference's order). One thread per segment: time-major columns
-// (coalesced across the segment threads) and segments of few steps.
+// (coalesced across the segment threads) and the segment-major ones seg_l1_tiled leaves.
 template <typename R, bool TM>
 __global__ void __launch_bounds__(256) k_seg_l1(const R* __restrict__ adv, long N, int T, double* __restrict__ L1) {
   const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -64,7 +60,7 @@ __global__ void __launch_bounds__(256) k_seg_l1(const R* __restrict__ adv, long 
 }
 // Segment-major: a block's 16 segments arrive 64 steps at a time in 64-wide runs (a thread per segment reads T
 // elements apart from its neighbours, on N / 64 wavefronts), and one lane per segment adds its row out of
-// LDS in order. 4096x64 f64: 6.1 -> 3.4 us.
+// LDS in order. 8192x64 f64: 5.1 -> 3.0 us.
 template <typename R>
 __global__ void __launch_bounds__(256) k_seg_l1_sm(const R* __restrict__ adv, long N, int T, double* __restrict__ L1) {
   __shared__ double tl[kSm][kSp];
@@ -572,7 +568,7 @@ int seg_l1(const ph_replay_cols& c, double* L1, hipStream_t st) {
   const long N = (long)c.N;
   const int T = (int)c.T;
   const unsigned g = ceil_div(c.N, 256), gs = ceil_div(c.N, kSm);
-  const bool tiles = sm_tiles(c);
+  const bool tiles = seg_l1_tiled(c.dtype == PH_F64, c.time_major, N, T);
   if (c.dtype == PH_F64) {
     if (tiles) k_seg_l1_sm<double><<<gs, 256, 0, st>>>((const double*)c.adv, N, T, L1);
     else if (c.time_major) k_seg_l1<double, true><<<g, 256, 0, st>>>((const double*)c.adv, N, T, L1);

@@ -62,4 +62,17 @@ inline bool vtrace_tiled(bool f64, bool time_major, long B, long T) {
   return B <= 24576 ? T >= 32 : B < 32768 && 2 * pad <= T;
 }
 
+// ---- Prioritised replay, segment-major columns ------------------------------------------------------------
+// The gather's tiles of 16 segments x 64 steps: rows of at least 16 steps (shorter ones fill too little of a 64-step
+// run, and a whole row is a cache line or less; 64 segments f64: T = 16 10.8 -> 8.9 us, 17 10.3 -> 9.1). The upper bound
+// keeps a tile's steps within int.
+inline bool gather_tiled(bool time_major, long T) { return !time_major && T >= 16 && T <= 1L << 30; }
+// The per-segment sums add one row per lane out of the tile, 16 lanes of a block at work: one thread per segment keeps
+// up while rows are short, and in fp32 while the segments are few (4096 segments, thread / tile: f64 T = 24 2.4 / 2.8
+// us, 32 3.4 / 2.6; fp32 32 2.6 / 2.7, 64 3.4 / 2.8; 65536 x 16 2.2 / 4.4; fp32 16 x 4096 55 / 62, 128 x 2048 35 / 33).
+inline bool seg_l1_tiled(bool f64, bool time_major, long N, long T) {
+  if (time_major || T > 1L << 30) return false;
+  return f64 ? T >= 32 : T >= 64 && N >= 128;
+}
+
 }  // namespace ph

@@ -23,7 +23,8 @@ def columns(N, T, K, np_dt, dt):
 
 @pytest.mark.parametrize("dtype", ["f64", "f32"])
 @pytest.mark.parametrize("N,T,B,K", [(1, 16, 1, 1), (40, 15, 17, 2), (40, 17, 16, 1), (15, 64, 15, 3), (33, 65, 100, 2),
-                                     (17, 130, 33, 1), (100, 520, 4096, 1)])
+                                     (17, 130, 33, 1), (100, 520, 4096, 1),
+                                     (128, 63, 5, 1), (129, 64, 20, 1), (127, 70, 9, 1), (20, 31, 9, 1), (20, 32, 9, 1)])
 def test_tiles(gpu, dtype, N, T, B, K):
     dt, np_dt, tol = DT[dtype]
     h, d = columns(N, T, K, np_dt, dt)

@@ -20,6 +20,8 @@ int main(int argc, char** argv) {
   if (!std::strcmp(argv[1], "fold_threads")) r = fold_threads((int)a[0], a[1]);
   if (!std::strcmp(argv[1], "sample_registers")) r = sample_registers(a[0]);
   if (!std::strcmp(argv[1], "vtrace_tiled")) r = vtrace_tiled(a[0], a[1], a[2], a[3]);
+  if (!std::strcmp(argv[1], "gather_tiled")) r = gather_tiled(a[0], a[1]);
+  if (!std::strcmp(argv[1], "seg_l1_tiled")) r = seg_l1_tiled(a[0], a[1], a[2], a[3]);
   std::printf("%ld\n", r);
   return 0;
 }
@@ -82,3 +84,16 @@ VTRACE = [(0, 1, 4096, 1, 0), (0, 1, 4096, 4, 0), (0, 1, 4096, 8, 1), (0, 1, 163
 @pytest.mark.parametrize("f64,tm,B,T,tiled", VTRACE)
 def test_vtrace_tiled(route, f64, tm, B, T, tiled):
     assert route("vtrace_tiled", f64, tm, B, T) == tiled
+
+
+@pytest.mark.parametrize("f64,N,T,tiled", [(0, 65536, 16, 0), (0, 4096, 24, 0), (0, 4096, 63, 0), (0, 4096, 64, 1), (0, 16, 4096, 0),
+                                           (0, 127, 2048, 0), (0, 128, 2048, 1), (1, 65536, 17, 0), (1, 4096, 24, 0),
+                                           (1, 4096, 32, 1), (1, 16, 4096, 1)])
+def test_seg_l1_tiled(route, f64, N, T, tiled):
+    assert route("seg_l1_tiled", f64, 0, N, T) == tiled
+    assert route("seg_l1_tiled", f64, 1, N, T) == 0
+
+
+@pytest.mark.parametrize("T,tiled", [(15, 0), (16, 1), (4096, 1)])
+def test_gather_tiled(route, T, tiled):
+    assert route("gather_tiled", 0, T) == tiled and route("gather_tiled", 1, T) == 0

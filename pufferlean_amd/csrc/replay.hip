@@ -8,8 +8,8 @@
 //   ph_mb_iterate   value/ratio of the sampled segments from the BPTT    (puffercuda.cu:503-511)
 //
 // Design: the reference chains seven launches for the sampler (weights, a one-block sum, a 64-chunk
-// single-thread scan, its combine and add, the draws). Here it is two: the segment weights, then blocks that
-// each form the fixed-tree sum and the cumulative table in their own LDS and take a share of the draws (one
+// single-thread scan, its combine and add, the draws). Here it is one for a few segments and draws, else two: the
+// segment weights, then blocks that each form the fixed-tree sum and the cumulative table in their own LDS and take a share of the draws (one
 // workgroup for everything once the table outgrows LDS). The gather is one pass that also produces per-block
 // (count, mean, M2) partials; the normalising kernel's blocks merge them in block order (Chan et al.'s
 // pairwise update), so mean and std cost no extra pass over the columns. Segment-major columns pass
@@ -98,16 +98,18 @@ __global__ void __launch_bounds__(256) k_seg_l1_sm(const R* __restrict__ adv, lo
 //   cum[e] = chunk-local running sum of p + the sum of the earlier chunks (fixed-tree scan)
 //   draw i: z = splitmix64 finaliser of rng + (i+1)*GOLD; u = (z >> 11) / 2^53 * total;
 //           idx = first e with cum[e] >= u (N-1 if none); mp[i] = exp(-beta * log(N * p[idx] + 1e-12))
-// In one workgroup the f64 exponentials and logarithms of the weights and the draws are what takes the time,
-// so they are spread over the chip: a kernel of weights, then (N up to kPsLdsCum) blocks of kPsDraws draws that
+// Past a few segments and draws (prio_one_block) the f64 exponentials and logarithms of the weights and the draws
+// are what takes the time in one workgroup, so they are spread over the chip: a kernel of weights, then (N up to kPsLdsCum) blocks of kPsDraws draws that
 // each form the table from the weights in their LDS, the same operations in the same order in every block.
-// 4096 segments, 4096 draws: 22.4 us in one workgroup, 2.6 + 8.4 in the two launches.
+// 4096 segments, 4096 draws: 21.9 us in one workgroup, 10.1 in the two launches.
 __device__ __forceinline__ double prio_p(double w, double denom) { return (w + 1e-6) / denom; }
+
+__device__ __forceinline__ double prio_weight(double l1, double alpha) { return exp(alpha * log(l1 + 1e-12)); }
 
 __global__ void __launch_bounds__(256) k_prio_weights(const double* __restrict__ L1, long N, double alpha,
                                                       double* __restrict__ w) {
   const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < N) w[e] = exp(alpha * log(L1[e] + 1e-12));
+  if (e < N) w[e] = prio_weight(L1[e], alpha);
 }
 
 // The cumulative table of the block's threads into cum; returns the total. red: kPsThreads doubles.
@@ -177,6 +179,20 @@ __global__ void __launch_bounds__(kPsThreads) k_prio_draws(const double* __restr
   const double total = prio_table(w, N, cum, red, denom);
   const long i = (long)blockIdx.x * kPsDraws + threadIdx.x;
   if (threadIdx.x < kPsDraws && i < B) prio_draw(i, cum, w, N, total, denom, beta, rng, seg, mp);
+}
+
+// prio_one_block: weights, table and draws in one launch of one workgroup, one segment per thread.
+constexpr long kPsOne = kPsThreads;
+__global__ void __launch_bounds__(kPsThreads) k_prio_one(const double* __restrict__ L1, long N, long B, double alpha,
+                                                         double beta, unsigned long long rng, int* __restrict__ seg,
+                                                         double* __restrict__ mp) {
+  __shared__ double red[kPsThreads];
+  __shared__ double w[kPsOne], cum[kPsOne];
+  for (long e = threadIdx.x; e < N; e += kPsThreads) w[e] = prio_weight(L1[e], alpha);
+  __syncthreads();
+  double denom;
+  const double total = prio_table(w, N, cum, red, denom);
+  for (long i = threadIdx.x; i < B; i += kPsThreads) prio_draw(i, cum, w, N, total, denom, beta, rng, seg, mp);
 }
 
 // More segments: one workgroup, the table in memory.
@@ -588,6 +604,12 @@ int prio_sample(const double* L1, size_t N, size_t B, double alpha, double beta,
   PH_REQUIRE(B <= 0x7fffffffUL, "prio_sample: %zu draws out of range", B);
   if (B == 0) return PH_OK;
   PH_REQUIRE(L1 && seg && mp, "prio_sample: null buffer");
+  if (prio_one_block((long)N, (long)B)) {
+    static_assert(kPsOne >= 1024, "segments of prio_one_block");
+    k_prio_one<<<1, kPsThreads, 0, st>>>(L1, (long)N, (long)B, alpha, beta, (unsigned long long)rng, seg, mp);
+    PH_LAUNCH_CHECK();
+    return PH_OK;
+  }
   const size_t tab = (N + 31) & ~(size_t)31;
   double* w = (double*)scratch(kSlotPrio, (N > (size_t)kPsLdsCum ? 2 : 1) * tab * 8);
   if (!w) return PH_ERR_NOMEM;

@@ -75,4 +75,9 @@ inline bool seg_l1_tiled(bool f64, bool time_major, long N, long T) {
   return f64 ? T >= 32 : T >= 64 && N >= 128;
 }
 
+// The sampler in one workgroup: few segments and draws, whose f64 functions are quick and where a second launch costs
+// more than they do (64 segments, 64 draws 5.6 us in one launch, 6.7 in two; 1024, 512 7.4 / 8.2; but 1024, 2048
+// 10.6 / 8.1 and 2048, 1024 10.2 / 8.8).
+inline bool prio_one_block(long N, long draws) { return N <= 1024 && draws <= 1024; }
+
 }  // namespace ph

@@ -1,6 +1,6 @@
 """Segment-major replay columns through the 16-segment x 64-step tiles: steps and draws around the tile's edges and
 the rule's limits, both types, several action components, repeated and invalid draws; and the sampler around the
-largest table it holds in LDS."""
+lines between its three forms."""
 import numpy as np
 import pytest
 import torch
@@ -89,7 +89,8 @@ def test_iterate_more_draws_than_the_pairwise_scan(gpu):
         assert np.array_equal(value.cpu().numpy(), ev)
 
 
-@pytest.mark.parametrize("N,B", [(8192, 1), (8192, 129), (8193, 129), (1024, 128), (1025, 127)])
+@pytest.mark.parametrize("N,B", [(8192, 1), (8192, 129), (8193, 129), (1024, 128), (1025, 127), (1, 5), (63, 1024),
+                                 (1024, 1024), (1000, 1025)])
 def test_sampler_edges(gpu, N, B):
     L1 = rng.randf(0x740 + N, N, 0.01, 5.0)
     seg, mp = D.prio_sample(torch.from_numpy(L1).cuda(), B, alpha=0.8, beta=0.2, rng_state=0x1234)

@@ -22,6 +22,7 @@ int main(int argc, char** argv) {
   if (!std::strcmp(argv[1], "vtrace_tiled")) r = vtrace_tiled(a[0], a[1], a[2], a[3]);
   if (!std::strcmp(argv[1], "gather_tiled")) r = gather_tiled(a[0], a[1]);
   if (!std::strcmp(argv[1], "seg_l1_tiled")) r = seg_l1_tiled(a[0], a[1], a[2], a[3]);
+  if (!std::strcmp(argv[1], "prio_one_block")) r = prio_one_block(a[0], a[1]);
   std::printf("%ld\n", r);
   return 0;
 }
@@ -97,3 +98,9 @@ def test_seg_l1_tiled(route, f64, N, T, tiled):
 @pytest.mark.parametrize("T,tiled", [(15, 0), (16, 1), (4096, 1)])
 def test_gather_tiled(route, T, tiled):
     assert route("gather_tiled", 0, T) == tiled and route("gather_tiled", 1, T) == 0
+
+
+@pytest.mark.parametrize("N,draws,one", [(1, 1, 1), (64, 64, 1), (1024, 1024, 1), (1025, 64, 0), (64, 1025, 0), (1024, 2048, 0),
+                                         (4096, 4096, 0)])
+def test_prio_one_block(route, N, draws, one):
+    assert route("prio_one_block", N, draws) == one

@@ -9,13 +9,13 @@
 //
 // Design: the reference chains seven launches for the sampler (weights, a one-block sum, a 64-chunk
 // single-thread scan, its combine and add, the draws). Here it is one for a few segments and draws, else two: the
-// segment weights, then blocks that each form the fixed-tree sum and the cumulative table in their own LDS and take a share of the draws (one
-// workgroup for everything once the table outgrows LDS). The gather is one pass that also produces per-block
+// segment weights, then blocks that each form the fixed-tree sum and the cumulative table in their own LDS and
+// take a share of the draws (one workgroup for them once the table outgrows LDS). The gather is one pass that also produces per-block
 // (count, mean, M2) partials; the normalising kernel's blocks merge them in block order (Chan et al.'s
 // pairwise update), so mean and std cost no extra pass over the columns. Segment-major columns pass
 // through LDS tiles of 16 segments x 64 steps, so that both the segment rows and the timestep-major
-// minibatch are read and written in runs. The iterate writes the last draw of a segment: found by comparing
-// the draws in each block, or for many draws through a last-writer table that the second launch leaves zeroed.
+// minibatch are read and written in runs. The iterate writes the last draw of a segment: found through a
+// last-writer table that the second launch leaves zeroed, or for long rows by comparing the draws in each block.
 //
 // Every reduction here has a fixed order, so results are reproducible run to run. They are not
 // bit-identical to the CPU twins, whose sums are sequential: mean, std, the probability normaliser
@@ -44,7 +44,6 @@ constexpr unsigned kFoldMax = 2048;  // gather blocks whose partials every norma
 constexpr int kSm = 16, kSt = 64;    // tile of segment-major columns: segments x steps
 constexpr int kSp = kSt + 1;         // its LDS pitch (a step of 16 segments hits distinct banks)
 inline bool sm_tiles(const ph_replay_cols& c) { return gather_tiled(c.time_major, (long)c.T); }
-constexpr long kScanDraws = 8192;    // draws compared pairwise by the segment-major iterate
 
 // ---- per-segment |adv| sums ------------------------------------------------------------------------
 // t ascending, f64 accumulation (the reference's order). One thread per segment: time-major columns
@@ -510,9 +509,9 @@ __global__ void __launch_bounds__(256) k_mb_iterate(R* __restrict__ value, R* __
   if (lane == 0) lw[e] = 0;
 }
 
-// Segment-major, up to kScanDraws draws: one launch. A block holds 16 draws, compares them with every later draw
-// (a draw whose segment is drawn again is not its last writer), and turns the timestep-major inputs of 64 steps
-// in LDS, so that a row's stores are 64-wide runs. 4096 draws x 64 f64: 9.0 us in two launches -> 8.2.
+// Segment-major, iterate_tiled: one launch, a block per 16 draws x 64 steps. It compares its draws with every later
+// draw (a draw whose segment is drawn again is not its last writer) and turns the timestep-major inputs in LDS, so that a
+// row's stores are 64-wide runs. The comparison runs while the tile's loads are in flight.
 template <typename R>
 __global__ void __launch_bounds__(256) k_mb_iterate_sm(R* __restrict__ value, R* __restrict__ ratio,
                                                        const R* __restrict__ logp, const float* __restrict__ newlp,
@@ -522,9 +521,20 @@ __global__ void __launch_bounds__(256) k_mb_iterate_sm(R* __restrict__ value, R*
   __shared__ int es[kSm];
   __shared__ unsigned again;  // bit k: draw b0 + k is not its segment's last
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const long b0 = (long)blockIdx.x * kSm;
+  const unsigned tiles = (unsigned)((T + kSt - 1) / kSt);
+  const long b0 = (long)(blockIdx.x / tiles) * kSm;
+  const int t0 = (int)(blockIdx.x % tiles) * kSt;
   if (tid < kSm) es[tid] = b0 + tid < B ? seg[b0 + tid] : -1;
   if (tid == 0) again = 0u;
+  const int ob = tid & (kSm - 1), ot = tid / kSm;
+  constexpr int kPer = kSt * kSm / 256;
+  float xl[kPer], xv[kPer];
+#pragma unroll
+  for (int k = 0; k < kPer; k++) {  // a step or draw past the end re-reads the last
+    const long os = (long)min(t0 + ot + k * (256 / kSm), T - 1) * B + min(b0 + ob, B - 1);
+    xl[k] = newlp[os];
+    xv[k] = newval[os];
+  }
   __syncthreads();
   int e[kSm];
 #pragma unroll
@@ -544,30 +554,21 @@ __global__ void __launch_bounds__(256) k_mb_iterate_sm(R* __restrict__ value, R*
       for (int k = 0; k < kSm; k++) hit |= (unsigned)(o[i] == e[k]) << k;
   }
   if (hit) atomicOr(&again, hit);
-  const int ob = tid & (kSm - 1), ot = tid / kSm;
-  for (int t0 = 0; t0 < T; t0 += kSt) {
-    __syncthreads();  // again is complete; the previous tile has been read
-    if (b0 + ob < B)
 #pragma unroll
-      for (int k = 0; k < kSt * kSm / 256; k++) {
-        const int u = ot + k * (256 / kSm);
-        if (t0 + u < T) {
-          const long os = (long)(t0 + u) * B + b0 + ob;
-          lp[ob][u] = newlp[os];
-          nv[ob][u] = newval[os];
-        }
-      }
-    __syncthreads();
-    if (t0 + lane < T)
-#pragma unroll
-      for (int k = 0; k < kSm / 4; k++) {
-        const int r = w + 4 * k;
-        if (es[r] < 0 || es[r] >= N || (again >> r & 1u)) continue;
-        const long si = (long)es[r] * T + t0 + lane;
-        ratio[si] = (R)exp((double)lp[r][lane] - (double)logp[si]);
-        value[si] = (R)nv[r][lane];
-      }
+  for (int k = 0; k < kPer; k++) {
+    lp[ob][ot + k * (256 / kSm)] = xl[k];
+    nv[ob][ot + k * (256 / kSm)] = xv[k];
   }
+  __syncthreads();
+  if (t0 + lane < T)
+#pragma unroll
+    for (int k = 0; k < kSm / 4; k++) {
+      const int r = w + 4 * k;
+      if (es[r] < 0 || es[r] >= N || (again >> r & 1u)) continue;
+      const long si = (long)es[r] * T + t0 + lane;
+      ratio[si] = (R)exp((double)lp[r][lane] - (double)logp[si]);
+      value[si] = (R)nv[r][lane];
+    }
 }
 
 int check_cols(const ph_replay_cols* c, const char* who) {
@@ -666,8 +667,8 @@ int mb_gather(const ph_replay_cols& c, const int* seg, const double* mp, size_t 
 int mb_iterate(const ph_replay_cols& c, const int* seg, size_t B, const float* newlp, const float* newval,
                hipStream_t st) {
   if (B == 0) return PH_OK;
-  if (sm_tiles(c) && B <= (size_t)kScanDraws) {
-    const unsigned g = ceil_div(B, kSm);
+  if (iterate_tiled(c.time_major, (long)B, (long)c.T)) {
+    const unsigned g = ceil_div(B, kSm) * ceil_div(c.T, kSt);
     if (c.dtype == PH_F64)
       k_mb_iterate_sm<double><<<g, 256, 0, st>>>((double*)c.value, (double*)c.ratio, (const double*)c.logp, newlp,
                                                  newval, seg, (long)B, (long)c.N, (int)c.T);

@@ -72,7 +72,7 @@ def test_tiles(gpu, dtype, N, T, B, K):
 
 
 def test_iterate_more_draws_than_the_pairwise_scan(gpu):
-    """One draw past the limit takes the last-writer table: the same values."""
+    """The most draws that may be compared pairwise and one more: the same values."""
     N, T = 60, 20
     h, d = columns(N, T, 1, np.float64, torch.float64)
     for B in (8192, 8193):
@@ -87,6 +87,28 @@ def test_iterate_more_draws_than_the_pairwise_scan(gpu):
         for e, b in last.items():
             ev[e] = newval.reshape(T, B)[:, b]
         assert np.array_equal(value.cpu().numpy(), ev)
+
+
+@pytest.mark.parametrize("N,T,B", [(60, 20, 8192), (60, 256, 8192), (60, 256, 8193), (300, 255, 40), (300, 257, 40),
+                                   (7, 130, 2047), (3000, 128, 2048), (50, 64, 8191), (50, 64, 8192), (5, 1000, 1)])
+def test_iterate_forms(gpu, N, T, B):
+    """Both sides of the rule between the tiles that compare draws and the last-writer table: the last draw of a
+    segment leaves its values, ratios to f64's exponential, other rows untouched; invalid draws are skipped."""
+    h, d = columns(N, T, 1, np.float64, torch.float64)
+    seg = rng.randint(0x730 + B, B, N)
+    if B > 20:
+        seg[[3, 17]] = [-1, N]
+    newlp, newval = rng.normal(0x731, T * B).astype(np.float32), rng.normal(0x732, T * B).astype(np.float32)
+    value, ratio = d["value"].clone(), torch.ones(N, T, device="cuda", dtype=torch.float64)
+    D.mb_iterate(D.ReplayColumns(N, T, value=value, ratio=ratio, logp=d["logp"]), torch.from_numpy(seg).to("cuda", torch.int32),
+                 torch.from_numpy(newlp).cuda(), torch.from_numpy(newval).cuda())
+    last = {int(e): b for b, e in enumerate(seg) if 0 <= e < N}
+    ev, er = h["value"].copy(), np.ones((N, T))
+    for e, b in last.items():
+        ev[e] = newval.reshape(T, B)[:, b]
+        er[e] = np.exp(newlp.reshape(T, B)[:, b].astype(np.float64) - h["logp"][e])
+    assert np.array_equal(value.cpu().numpy(), ev)
+    np.testing.assert_allclose(ratio.cpu().numpy(), er, rtol=1e-15)
 
 
 @pytest.mark.parametrize("N,B", [(8192, 1), (8192, 129), (8193, 129), (1024, 128), (1025, 127), (1, 5), (63, 1024),

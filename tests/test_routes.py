@@ -23,6 +23,7 @@ int main(int argc, char** argv) {
   if (!std::strcmp(argv[1], "gather_tiled")) r = gather_tiled(a[0], a[1]);
   if (!std::strcmp(argv[1], "seg_l1_tiled")) r = seg_l1_tiled(a[0], a[1], a[2], a[3]);
   if (!std::strcmp(argv[1], "prio_one_block")) r = prio_one_block(a[0], a[1]);
+  if (!std::strcmp(argv[1], "iterate_tiled")) r = iterate_tiled(a[0], a[1], a[2]);
   std::printf("%ld\n", r);
   return 0;
 }
@@ -104,3 +105,10 @@ def test_gather_tiled(route, T, tiled):
                                          (4096, 4096, 0)])
 def test_prio_one_block(route, N, draws, one):
     assert route("prio_one_block", N, draws) == one
+
+
+@pytest.mark.parametrize("draws,T,tiled", [(64, 16, 0), (64, 64, 0), (4096, 16, 0), (8192, 16, 0), (8192, 32, 0), (4096, 64, 0),
+                                           (4096, 65, 0), (1024, 128, 0), (2048, 128, 1), (8192, 64, 1), (16, 256, 1),
+                                           (4096, 256, 1), (8193, 256, 0)])
+def test_iterate_tiled(route, draws, T, tiled):
+    assert route("iterate_tiled", 0, draws, T) == tiled and route("iterate_tiled", 1, draws, T) == 0

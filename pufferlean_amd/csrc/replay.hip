@@ -40,7 +40,6 @@ constexpr int kPsDraws = 128;     // draws per block of the LDS sampler
 constexpr int kGaThreads = 256;
 constexpr int kGaPer = 4;         // minibatch elements per gather thread (256 blocks at 4096 x 64)
 constexpr int kGaBlock = kGaThreads * kGaPer;
-constexpr unsigned kFoldMax = 2048;  // gather blocks whose partials every normalising block merges itself
 constexpr int kSm = 16, kSt = 64;    // tile of segment-major columns: segments x steps
 constexpr int kSp = kSt + 1;         // its LDS pitch (a step of 16 segments hits distinct banks)
 inline bool sm_tiles(const ph_replay_cols& c) { return gather_tiled(c.time_major, (long)c.T); }
@@ -259,8 +258,8 @@ __device__ inline void block_moments(double (&sh)[3][kGaThreads], double s, int 
 //   act (K wide, truncated to an integer) | adv (raw here) | ret = adv + value | old = logp |
 //   term = term > 0.5 ? 1 : 0 | ov = value
 // An index outside [0, N) yields NaN columns for that row (the sampler never produces one).
-// Each block also reduces its raw adv values to (count, mean, M2) in part; k_mb_stats merges the
-// blocks in index order into stats = [mean, std] (population std).
+// Each block also reduces its raw adv values to (count, mean, M2) in part; the normalising kernel (or k_mb_stats,
+// past gather_folds) merges the blocks in index order into stats = [mean, std] (population std).
 template <typename R, bool TM>
 __global__ void __launch_bounds__(kGaThreads) k_mb_gather(
     const R* __restrict__ adv, const R* __restrict__ value, const R* __restrict__ act,
@@ -436,8 +435,8 @@ __global__ void __launch_bounds__(kGaThreads) k_mb_stats(const double* __restric
 }
 
 // adv[j] = mp[bi] * (adv[j] - mean) / (std + 1e-8), j = t*B + bi (mp NULL: weight 1). FOLD: every block merges
-// the gather's partials itself (up to kFoldMax of them: the merge costs less than a launch of one block:
-// 4.0 + 2.8 -> 4.9 us), and the first writes stats; else stats are given.
+// the gather's partials itself (gather_folds: the merge costs less than a launch of one block), and the first
+// writes stats; else stats are given.
 template <typename R, bool FOLD>
 __global__ void __launch_bounds__(kGaThreads) k_mb_normalize(R* __restrict__ adv, long B, long n,
                                                              const double* __restrict__ mp,
@@ -639,7 +638,7 @@ int mb_gather(const ph_replay_cols& c, const int* seg, const double* mp, size_t 
   }
   const long N = (long)c.N;
   const int T = (int)c.T;
-  const bool fold = nb <= kFoldMax;
+  const bool fold = gather_folds(nb);
 #define PH_GATHER_ARGS(R)                                                                                          \
   (const R*)c.adv, (const R*)c.value, (const R*)c.act, (const R*)c.logp, (const R*)c.term, N, T, K, seg, (long)B, \
       (R*)out, part

@@ -67,6 +67,10 @@ inline bool vtrace_tiled(bool f64, bool time_major, long B, long T) {
 // run, and a whole row is a cache line or less; 64 segments f64: T = 16 10.8 -> 8.9 us, 17 10.3 -> 9.1). The upper bound
 // keeps a tile's steps within int.
 inline bool gather_tiled(bool time_major, long T) { return !time_major && T >= 16 && T <= 1L << 30; }
+// Gather blocks whose (count, mean, M2) partials every normalising block merges itself; past that a launch of one block
+// does (1024 partials, time-major f64 256 draws x 4096: merged by every block 25.8 us, by one 26.9; 2048, 4096 x 512:
+// 78.0 and 76.0, fp32 1024 x 2048 42.1 and 39.6).
+inline bool gather_folds(long blocks) { return blocks <= 1024; }
 // The per-segment sums add one row per lane out of the tile, 16 lanes of a block at work: one thread per segment keeps
 // up while rows are short, and in fp32 while the segments are few (4096 segments, thread / tile: f64 T = 24 2.4 / 2.8
 // us, 32 3.4 / 2.6; fp32 32 2.6 / 2.7, 64 3.4 / 2.8; 65536 x 16 2.2 / 4.4; fp32 16 x 4096 55 / 62, 128 x 2048 35 / 33).

@@ -24,6 +24,7 @@ int main(int argc, char** argv) {
   if (!std::strcmp(argv[1], "seg_l1_tiled")) r = seg_l1_tiled(a[0], a[1], a[2], a[3]);
   if (!std::strcmp(argv[1], "prio_one_block")) r = prio_one_block(a[0], a[1]);
   if (!std::strcmp(argv[1], "iterate_tiled")) r = iterate_tiled(a[0], a[1], a[2]);
+  if (!std::strcmp(argv[1], "gather_folds")) r = gather_folds(a[0]);
   std::printf("%ld\n", r);
   return 0;
 }
@@ -112,3 +113,8 @@ def test_prio_one_block(route, N, draws, one):
                                            (4096, 256, 1), (8193, 256, 0)])
 def test_iterate_tiled(route, draws, T, tiled):
     assert route("iterate_tiled", 0, draws, T) == tiled and route("iterate_tiled", 1, draws, T) == 0
+
+
+@pytest.mark.parametrize("blocks,folds", [(1, 1), (1024, 1), (1025, 0), (2048, 0)])
+def test_gather_folds(route, blocks, folds):
+    assert route("gather_folds", blocks) == folds

@@ -10,8 +10,8 @@
 // The step runs the encoder (bias fused) on the MFMA GEMM, then one kernel per layer that forms a unit's hid,
 // gate and proj products in one wavefront's accumulators and applies the cell to them in registers, and one
 // kernel for the head (action logits and the value, bias fused, written straight into the [N][A+1]
-// output). Hidden sizes that are no multiple of 8 run the products on the GEMM, a cell kernel and a padded
-// head instead.
+// output). Hidden sizes that are no multiple of 8, and the large ones rollout_form leaves, run the products on the
+// GEMM, a cell kernel and a padded head instead.
 // Its launches are plain stream work, so a caller can capture a whole horizon in one HIP graph.
 #include <cmath>
 #include <type_traits>
@@ -169,8 +169,8 @@ __device__ __forceinline__ float cell(float hid, float gate, float proj, float p
 // and the 32 units, so the cell runs on its accumulators and the [N][3H] products never reach memory (they were
 // 50 MB of a 4096 x 512 step's traffic, and the cell a launch of 10.6 us). X: the layer input in the
 // product's type (bf16 copy or fp32), xin the same in fp32 for the cell's skip; the fp32 weights are rounded on
-// their way into LDS. Bound by operand delivery into the CUs (256 rows x 96 weight rows a block, one block
-// per CU at 4096 x 512); two k chunks in flight in registers, LDS double-buffered.
+// their way into LDS. Operands into the CUs are what a block moves most of (256 rows x 96 weight rows, one block
+// per CU at 4096 x 512); two k chunks in flight in registers, LDS double-buffered. rollout_form chooses NW.
 // 4096 rows, H 512: 19.9 + 10.6 us -> about 22 (bf16 products); the whole step 89 -> 59 us, fp32 208 -> 157.
 template <bool BF, int NW>
 __global__ void __launch_bounds__(64 * NW, 1) k_roll_layer(const void* __restrict__ X, const float* __restrict__ xin,
@@ -439,27 +439,26 @@ int sample_actions(int dtype, const void* Y, size_t ldy, size_t N, size_t A, int
   return PH_OK;
 }
 
-// Layer tiles: 256 rows a block (one block per CU and the fewest weight re-reads) once that fills most CUs
-// (a step of 4096 rows, H 512, L 2: 59 us, against 76 with 128 rows), 128 rows from half of that (2048 rows:
-// 44 us), else 32-row blocks with k split over their wavefronts (48 to 1024 rows: 14 to 45 us, the unfused step
-// 17 to 54).
 template <bool BF>
-void launch_layer(const void* X, const float* xin, const float* W, float* state, float* xout, uint16_t* xoutb, long N,
-                  int L, int H, int l, hipStream_t st) {
+void launch_layer(RollForm form, const void* X, const float* xin, const float* W, float* state, float* xout,
+                  uint16_t* xoutb, long N, int L, int H, int l, hipStream_t st) {
   const unsigned gj = ceil_div(H, 32);
-  const long b256 = ((N + 255) / 256) * gj;
-  if (b256 >= 192)
-    k_roll_layer<BF, 8><<<dim3(ceil_div(N, 256), gj), 512, 0, st>>>(X, xin, W, state, xout, xoutb, N, L, H, l);
-  else if (b256 >= 96)
-    k_roll_layer<BF, 4><<<dim3(ceil_div(N, 128), gj), 256, 0, st>>>(X, xin, W, state, xout, xoutb, N, L, H, l);
-  else
+  if (form == kRoll32) {
     k_roll_reg<BF, 3><<<dim3(ceil_div(N, 32), gj), 256, 0, st>>>(X, xin, W, nullptr, nullptr, nullptr, state, xout,
                                                                  xoutb, N, L, H, l, 0);
+    return;
+  }
+  if constexpr (BF)
+    if (form == kRoll256) {
+      k_roll_layer<BF, 8><<<dim3(ceil_div(N, 256), gj), 512, 0, st>>>(X, xin, W, state, xout, xoutb, N, L, H, l);
+      return;
+    }
+  k_roll_layer<BF, 4><<<dim3(ceil_div(N, 128), gj), 256, 0, st>>>(X, xin, W, state, xout, xoutb, N, L, H, l);
 }
 
 template <bool BF>
-int rollout_fused(const ph_mingru_dims& d, const float* params, const float* obs, float* state, float* out,
-                  hipStream_t st) {
+int rollout_fused(RollForm form, const ph_mingru_dims& d, const float* params, const float* obs, float* state,
+                  float* out, hipStream_t st) {
   const long N = d.B;
   const int D = d.D, H = d.H, L = d.L, A = d.A;
   const size_t nx = ((size_t)N * H + 63) & ~(size_t)63;
@@ -478,7 +477,7 @@ int rollout_fused(const ph_mingru_dims& d, const float* params, const float* obs
   const float* wl = params + (long)H * D + H;
   auto in = [&](int i) { return BF ? (const void*)xb[i] : (const void*)x[i]; };
   for (int l = 0; l < L; l++) {
-    launch_layer<BF>(in(l & 1), x[l & 1], wl + (long)l * 3 * H * H, state, x[(l + 1) & 1], xb[(l + 1) & 1], N, L, H, l,
+    launch_layer<BF>(form, in(l & 1), x[l & 1], wl + (long)l * 3 * H * H, state, x[(l + 1) & 1], xb[(l + 1) & 1], N, L, H, l,
                      st);
     PH_LAUNCH_CHECK();
   }
@@ -497,9 +496,11 @@ int mingru_rollout_step(const ph_mingru_dims& d, const float* params, const floa
   // the fused kernels read weight rows and layer inputs in 16- and 32-byte pieces along k: whole pieces need
   // H a multiple of 8, and 16-byte alignment of the layers' rows (they start at H D + H floats, then a
   // multiple of 8; the head's value row may sit at any offset and is read with 4-byte alignment).
-  if (H % 8 == 0 && ((uintptr_t)params & 15) == 0)
-    return d.precision ? rollout_fused<false>(d, params, obs, state, out, st)
-                       : rollout_fused<true>(d, params, obs, state, out, st);
+  const RollForm form =
+      H % 8 == 0 && ((uintptr_t)params & 15) == 0 ? rollout_form(!d.precision, N, H) : kRollChain;
+  if (form != kRollChain)
+    return d.precision ? rollout_fused<false>(form, d, params, obs, state, out, st)
+                       : rollout_fused<true>(form, d, params, obs, state, out, st);
   const size_t nx = (size_t)N * H;
   float* base = (float*)scratch(kSlotRollout, (2 * nx + (size_t)N * 3 * H + (size_t)HP * H + HP) * 4);
   if (!base) return PH_ERR_NOMEM;

@@ -96,4 +96,36 @@ inline bool iterate_tiled(bool time_major, long draws, long T) {
   return T >= 256 || (T >= 128 && n >= 1L << 18) || (T >= 64 && n >= 1L << 19);
 }
 
+// ---- MinGRU rollout step ----------------------------------------------------------------------------------
+// The layer kernel of N rows and H units (H a multiple of 8): blocks of 32 rows with k split over the wavefronts, of
+// 128 or 256 rows with the weights in LDS, or the GEMM chain (products, a cell kernel, a padded head).
+// A launch takes rounds of as many blocks as run at a time, and a round costs about the same however full: bf16
+// products, bound by operand delivery, 256 blocks of any form, a round of 32 / 128 / 256 rows costing about 10 / 18 / 23
+// (below 320 units 10 / 28 / 36; steps of two layers, 512 units: 512 rows 31 / 38 / 44 us, 700 44 / 40 / 45, 2048 71 /
+// 42 / 48, 4096 126 / 74 / 57, chain 88; 384: 1500 58 / 37 / 43, chain 46). Past 1280 units few rows go to the chain,
+// whose split k keeps the chip busy (2048 units, 48 rows 75, chain 60; 200 rows 128-row blocks 82, chain 100).
+// fp32 products, bound by the matrix core, 768 blocks of 32 rows or 256 of 128, a round of either about as long; 256-row
+// blocks are never the faster form. Past 512 units the chain's 128x128 tiles fill their rounds better at some
+// sizes (in units of a round: 9 per round of 128-row blocks + 3, 11 per round of chain tiles + 5.5; 768 units: 2600
+// rows 204, chain 264; 3300 294, chain 274), and past 768 the chain takes the few rows (896: 256 rows 92, chain 95; 300
+// 101, chain 95; 1024: 100 rows 100, chain 94, but 1024 rows in 128-row blocks 165, chain 203).
+enum RollForm { kRollChain = 0, kRoll32, kRoll128, kRoll256 };
+inline RollForm rollout_form(bool bf16, long N, long H) {
+  const auto up = [](long a, long b) { return (a + b - 1) / b; };
+  const long cols = up(H, 32), b32 = up(N, 32) * cols, b128 = up(N, 128) * cols, b256 = up(N, 256) * cols;
+  if (bf16) {
+    if (H > 2048 || (H > 1280 && N <= 128)) return kRollChain;
+    const long c32 = 10 * up(b32, 256), c128 = (H >= 320 ? 18 : 28) * up(b128, 256),
+               c256 = (H >= 320 ? 23 : 36) * up(b256, 256);
+    if (c32 <= c128 && c32 <= c256) return kRoll32;
+    return c128 <= c256 ? kRoll128 : kRoll256;
+  }
+  if (H > 2048) return kRollChain;
+  if (H > 768 && N <= 768) return H <= 896 && N <= 256 ? kRoll32 : kRollChain;
+  const long r32 = up(b32, 768), r128 = up(b128, 256), chain = up(up(N, 128) * up(3 * H, 128), 256);
+  if (H > 512 && (r128 >= 2 || H > 768) && 18 * r128 + 6 >= 22 * chain + 11) return kRollChain;
+  if (H > 768) return kRoll128;
+  return r32 <= r128 ? kRoll32 : kRoll128;
+}
+
 }  // namespace ph

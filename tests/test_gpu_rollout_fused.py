@@ -64,6 +64,15 @@ def test_step(D, N, H, A, L, precision):
     assert bool((guard[N:] == 7.0).all())
 
 
+# both sides of the lines between the forms: 700 and 2600 rows of 512 units, few rows of 1280 and more, fp32 past 768
+# units and where the chain's tiles fill their rounds
+@pytest.mark.parametrize("N,H", [(700, 512), (2600, 512), (33, 1288), (129, 1288), (3, 2056), (256, 776), (257, 776), (40, 904),
+                                 (300, 320), (3300, 768)])
+@pytest.mark.parametrize("precision", [0, 1])
+def test_step_forms(D, N, H, precision):
+    test_step(D, N, H, 6, 1, precision)
+
+
 @pytest.mark.parametrize("dt", [torch.float32, torch.float64])
 @pytest.mark.parametrize("A", [1, 2, 4, 5, 8, 9, 15, 16, 17, 32, 33])
 def test_sampler_widths(D, A, dt):

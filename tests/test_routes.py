@@ -25,6 +25,7 @@ int main(int argc, char** argv) {
   if (!std::strcmp(argv[1], "prio_one_block")) r = prio_one_block(a[0], a[1]);
   if (!std::strcmp(argv[1], "iterate_tiled")) r = iterate_tiled(a[0], a[1], a[2]);
   if (!std::strcmp(argv[1], "gather_folds")) r = gather_folds(a[0]);
+  if (!std::strcmp(argv[1], "rollout_form")) r = rollout_form(a[0], a[1], a[2]);
   std::printf("%ld\n", r);
   return 0;
 }
@@ -118,3 +119,18 @@ def test_iterate_tiled(route, draws, T, tiled):
 @pytest.mark.parametrize("blocks,folds", [(1, 1), (1024, 1), (1025, 0), (2048, 0)])
 def test_gather_folds(route, blocks, folds):
     assert route("gather_folds", blocks) == folds
+
+
+# (bf16, rows, units) and the faster form: 0 the GEMM chain, 1, 2 and 3 blocks of 32, 128 and 256 rows
+ROLLOUT = [(1, 48, 128, 1), (1, 2048, 128, 1), (1, 16384, 128, 3), (1, 4096, 256, 2), (1, 6000, 256, 3), (1, 512, 512, 1),
+           (1, 700, 512, 2), (1, 2048, 512, 2), (1, 2600, 512, 3), (1, 4096, 512, 3), (1, 1500, 384, 2), (1, 3300, 384, 3),
+           (1, 1024, 640, 2), (1, 300, 1024, 2), (1, 2600, 768, 2), (1, 200, 1280, 2), (1, 48, 2048, 0), (1, 200, 2048, 2),
+           (1, 48, 4096, 0), (0, 48, 128, 1), (0, 8192, 128, 2), (0, 2048, 384, 1), (0, 1300, 512, 1), (0, 2048, 512, 2),
+           (0, 4096, 512, 2), (0, 6000, 256, 1), (0, 4096, 640, 0), (0, 2600, 768, 2), (0, 3300, 768, 0), (0, 48, 896, 1),
+           (0, 300, 896, 0), (0, 700, 896, 0), (0, 1, 1024, 0), (0, 1024, 1024, 2), (0, 2600, 1024, 0), (0, 48, 2048, 0),
+           (0, 2048, 1280, 0), (0, 1024, 2048, 2), (0, 1024, 2056, 0)]
+
+
+@pytest.mark.parametrize("bf,N,H,form", ROLLOUT)
+def test_rollout_form(route, bf, N, H, form):
+    assert route("rollout_form", bf, N, H) == form

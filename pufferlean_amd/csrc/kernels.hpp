@@ -160,13 +160,8 @@ int ns_fused(float* const* X, const int* rows, const int* cols, int n, const flo
 size_t ns_fused_ws_bytes(int rows, int cols, int nsteps);
 
 // fp32-MFMA Newton-Schulz of a batch, one launch per phase for up to kNsMaxMats matrices (more run as
-// further launches), each of a shape ns_f32_fits accepts; ws_slot as above. The GEMM chain keeps the rest: a
-// tile's k loop is not split over blocks, so a side past 2048 leaves one chain of over 7 us per phase, and
-// 32x32 tiles re-read their operands too often once there are thousands of them (5 steps, batched launches
-// against chain: 2048x64 141 against 234 us, 1536x1536 1.22 against 2.01 ms, 2048x2048 2.69 against 2.64).
-inline bool ns_f32_fits(int rows, int cols) {
-  return rows <= 2048 && cols <= 2048 && (long)rows * cols <= 3L << 20;
-}
+// further launches), each of a shape ns_f32_fits (routes.hpp) accepts; ws_slot as above. The GEMM chain keeps the
+// rest.
 int ns_f32_batch(float* const* X, const int* rows, const int* cols, int n, const float* coeffs, int nsteps, float eps,
                  int ws_slot, hipStream_t st);
 

@@ -12,6 +12,7 @@
 //    Tall matrices are transposed to wide on the way in and back on the way out.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "routes.hpp"
 
 namespace ph {
 namespace {

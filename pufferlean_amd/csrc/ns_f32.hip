@@ -18,6 +18,7 @@
 // 419 -> 227, 768x768 404 -> 293; four matrices of a small policy (288x96, 96x40, 5x96, 1x96) 270 -> 86.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "routes.hpp"
 
 namespace ph {
 namespace {

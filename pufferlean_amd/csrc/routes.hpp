@@ -96,6 +96,20 @@ inline bool iterate_tiled(bool time_major, long draws, long T) {
   return T >= 256 || (T >= 128 && n >= 1L << 18) || (T >= 64 && n >= 1L << 19);
 }
 
+// ---- Newton-Schulz in fp32 ----------------------------------------------------------------------------------
+// Whether a matrix takes the batched launches of 32x32 tiles (one per phase) or the GEMM chain. By its shape alone, so that
+// a matrix gives the same result alone and in a batch. A tile's k loop is not split over blocks, so a side past 2048
+// leaves one chain of over 7 us per phase, and 32x32 tiles re-read their operands too often once there are thousands of
+// them (5 steps, chain / launches: 2048x64 234 / 133 us, 1536x1536 2014 / 1219, 2048x1536 2215 / 1480, but 2048x2048
+// 2640 / 2690). Around 1024x1024 the chain's products are 64 whole 128x128 tiles, so two or three matrices run side by side
+// on their streams: one 510 / 483 us, two 750 / 810, three 970 / 1132; from 1152 on it does not keep up (one 812 / 623,
+// two 1165 / 1108). Four of a size depend on how the runtime maps the side streams to hardware queues (four 1536x1536
+// 4093 or 5433 / 4441).
+inline bool ns_f32_fits(int rows, int cols) {
+  const int lo = rows < cols ? rows : cols, hi = rows < cols ? cols : rows;
+  return hi <= 2048 && (long)lo * hi <= 3L << 20 && !(lo >= 1024 && hi < 1152);
+}
+
 // ---- MinGRU rollout step ----------------------------------------------------------------------------------
 // The layer kernel of N rows and H units (H a multiple of 8): blocks of 32 rows with k split over the wavefronts, of
 // 128 or 256 rows with the weights in LDS, or the GEMM chain (products, a cell kernel, a padded head).

@@ -46,3 +46,18 @@ def test_ns_f32_batch_equals_single_calls(gpu):
         one = torch.from_numpy(m).cuda()
         D.newton_schulz(one, coeffs=O.REF_COEFFS, math="f32")
         assert torch.equal(one, b), m.shape
+
+
+@pytest.mark.parametrize("shape", [(1023, 1024), (1024, 1024)])
+def test_ns_f32_large_alone_and_in_a_batch(gpu, shape):
+    """The last shape of the launches and the first of the chain near 1024: the f64 iteration's result, and in a batch of
+    four the same bits as alone."""
+    x0 = rng.normal(0x700 + shape[0], shape[0] * shape[1], 0.0, 0.02).reshape(shape).astype(np.float32)
+    one = torch.from_numpy(x0).cuda()
+    D.newton_schulz(one, coeffs=O.REF_COEFFS, math="f32")
+    ref = ns64(x0.astype(np.float64), O.REF_COEFFS)
+    assert np.linalg.norm(one.cpu().numpy() - ref) <= TOL * np.linalg.norm(ref)
+    batch = [torch.from_numpy(x0).cuda() for _ in range(4)] + [torch.from_numpy(x0[:60, :90].copy()).cuda()]
+    D.newton_schulz_batch(batch, coeffs=O.REF_COEFFS, math="f32")
+    for b in batch[:4]:
+        assert torch.equal(b, one)

@@ -26,6 +26,7 @@ int main(int argc, char** argv) {
   if (!std::strcmp(argv[1], "iterate_tiled")) r = iterate_tiled(a[0], a[1], a[2]);
   if (!std::strcmp(argv[1], "gather_folds")) r = gather_folds(a[0]);
   if (!std::strcmp(argv[1], "rollout_form")) r = rollout_form(a[0], a[1], a[2]);
+  if (!std::strcmp(argv[1], "ns_f32_fits")) r = ns_f32_fits((int)a[0], (int)a[1]);
   std::printf("%ld\n", r);
   return 0;
 }
@@ -134,3 +135,10 @@ ROLLOUT = [(1, 48, 128, 1), (1, 2048, 128, 1), (1, 16384, 128, 3), (1, 4096, 256
 @pytest.mark.parametrize("bf,N,H,form", ROLLOUT)
 def test_rollout_form(route, bf, N, H, form):
     assert route("rollout_form", bf, N, H) == form
+
+
+@pytest.mark.parametrize("rows,cols,fits", [(512, 512, 1), (1023, 1023, 1), (2048, 1023, 1), (2048, 64, 1), (1023, 1100, 1),
+                                            (1024, 1024, 0), (1100, 1151, 0), (1024, 1152, 1), (1152, 1024, 1),
+                                            (1536, 1536, 1), (2048, 1536, 1), (2048, 1537, 0), (2049, 8, 0), (8, 2049, 0)])
+def test_ns_f32_fits(route, rows, cols, fits):
+    assert route("ns_f32_fits", rows, cols) == fits

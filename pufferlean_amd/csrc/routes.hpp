@@ -87,13 +87,13 @@ inline bool prio_one_block(long N, long draws) { return N <= 1024 && draws <= 10
 // The value / ratio iterate: tiles of 16 draws x 64 steps that compare their draws with every later one, in one launch,
 // or two launches through a last-writer table with a wavefront per draw. The comparison costs each block a pass
 // over the draws (so a bound on them), the table a launch; a wavefront per draw reads B apart in the timestep-major
-// inputs and is one chain over T. f64, table / tiles: 64 draws of 64 steps 4.2 / 5.1 us, 4096 of 16 5.0 / 6.4, 4096 of
-// 64 6.1 / 6.5, 1024 of 128 5.1 / 5.2, 2048 of 128 6.0 / 5.5, 8192 of 64 10.9 / 9.2, 256 of 256 5.2 / 5.1, 16 of 1024
-// 8.0 / 4.0, 4096 of 256 21.8 / 10.1.
+// inputs and is one chain over T. f64, table / tiles, over twenty sets of columns in turn (an update's columns are new
+// to the L2): 64 draws of 64 steps 4.1 / 5.2 us, 4096 of 16 6.0 / 7.0, 4096 of 32 7.1 / 7.5, 1024 of 64 5.7 / 5.7, 4096 of
+// 64 9.1 / 7.6, 256 of 128 5.9 / 5.4, 512 of 256 8.1 / 6.3, 4096 of 128 13.5 / 8.3; 16 of 1024 8.0 / 4.0. (The same set
+// again and again, the L2 warm: 4096 of 64 6.1 / 6.5, 1024 of 128 5.1 / 5.2, 4096 of 256 21.8 / 10.1.)
 inline bool iterate_tiled(bool time_major, long draws, long T) {
   if (time_major || draws > 8192 || T > 1L << 30) return false;
-  const long n = draws * T;
-  return T >= 256 || (T >= 128 && n >= 1L << 18) || (T >= 64 && n >= 1L << 19);
+  return T >= 256 || (T >= 128 && draws >= 256) || (T >= 64 && draws >= 1024);
 }
 
 // ---- Newton-Schulz in fp32 ----------------------------------------------------------------------------------

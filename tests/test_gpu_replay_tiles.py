@@ -90,7 +90,7 @@ def test_iterate_more_draws_than_the_pairwise_scan(gpu):
 
 
 @pytest.mark.parametrize("N,T,B", [(60, 20, 8192), (60, 256, 8192), (60, 256, 8193), (300, 255, 40), (300, 257, 40),
-                                   (7, 130, 2047), (3000, 128, 2048), (50, 64, 8191), (50, 64, 8192), (5, 1000, 1)])
+                                   (7, 130, 255), (3000, 128, 256), (50, 64, 1023), (50, 65, 1024), (50, 64, 8192), (5, 1000, 1)])
 def test_iterate_forms(gpu, N, T, B):
     """Both sides of the rule between the tiles that compare draws and the last-writer table: the last draw of a
     segment leaves its values, ratios to f64's exponential, other rows untouched; invalid draws are skipped."""

@@ -110,9 +110,9 @@ def test_prio_one_block(route, N, draws, one):
     assert route("prio_one_block", N, draws) == one
 
 
-@pytest.mark.parametrize("draws,T,tiled", [(64, 16, 0), (64, 64, 0), (4096, 16, 0), (8192, 16, 0), (8192, 32, 0), (4096, 64, 0),
-                                           (4096, 65, 0), (1024, 128, 0), (2048, 128, 1), (8192, 64, 1), (16, 256, 1),
-                                           (4096, 256, 1), (8193, 256, 0)])
+@pytest.mark.parametrize("draws,T,tiled", [(64, 16, 0), (64, 64, 0), (4096, 16, 0), (8192, 16, 0), (8192, 32, 0), (4096, 63, 0),
+                                           (1023, 64, 0), (1024, 64, 1), (4096, 64, 1), (8192, 64, 1), (255, 128, 0),
+                                           (256, 128, 1), (16, 256, 1), (4096, 256, 1), (8193, 256, 0)])
 def test_iterate_tiled(route, draws, T, tiled):
     assert route("iterate_tiled", 0, draws, T) == tiled and route("iterate_tiled", 1, draws, T) == 0
 

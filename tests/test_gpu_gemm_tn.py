@@ -98,3 +98,37 @@ def test_fold_forms(D, M, N, splits, cdt):
     ref = a.double().t() @ b.double()
     err = ((out.double() - ref).norm() / ref.norm()).item()
     assert err < (1e-5 if cdt == torch.float32 else 2 ** -8)
+
+
+@pytest.mark.parametrize("M,N,K", [(136, 200, 4097), (128, 256, 5001), (512, 512, 131079), (264, 136, 262147), (8192, 2048, 77)],
+                         ids=["128x256", "128x256-ragged-splits", "256x256-dma", "256x256-dma-ragged-tile", "256x128"])
+def test_tn_any_k_large_tiles(D, M, N, K):
+    """The bf16 kernels of the large weight gradients with a reduction that ends inside a k-tile: 128x256 splits, the
+    load-to-LDS kernel at 256x256 and the unsplit 256x128 tiles. Rows past the end hold NaN."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = (torch.full((K + 40, n), float("nan"), device="cuda", dtype=torch.bfloat16) for n in (M, N))
+    for x in (a, b):
+        x[:K] = torch.randn(K, x.shape[1], generator=g, device="cuda").bfloat16()
+    print(f"TN {M}x{N}x{K}", flush=True)
+    out = D.gemm(a[:K], b[:K], trans_a=True)
+    ref = torch.zeros(M, N, device="cuda", dtype=torch.float64)
+    for k0 in range(0, K, 32768):
+        ref += a[k0:min(K, k0 + 32768)].double().t() @ b[k0:min(K, k0 + 32768)].double()
+    assert ((out.double() - ref).norm() / ref.norm()).item() < 1e-5
+
+
+@pytest.mark.parametrize("M,N,K", [(136, 40, 4099), (40, 64, 9001), (304, 96, 999), (256, 256, 4101)])
+def test_tn_any_k_split_bf16(D, M, N, K):
+    """Split-bf16 products of a ragged reduction. Each operand is held to 2^-17 of its value and the product of the two low
+    halves (2^-18) is dropped: 2.5 x 2^-17 and the fp32 sums' 1e-5."""
+    from pufferlean_amd import _lib as L
+    g = torch.Generator(device="cuda").manual_seed(K)
+    a, b = (torch.full((K + 8, n), float("nan"), device="cuda") for n in (M, N))
+    for x in (a, b):
+        x[:K] = torch.randn(K, x.shape[1], generator=g, device="cuda")
+    out = torch.empty(M, N, device="cuda")
+    p = lambda x: D._p(x)
+    L.call("ph_gemm", 1, 0, M, N, K, L.PH_F32, p(a), M, L.PH_F32, p(b), N, L.PH_F32, p(out), N, L.PH_MATH_BF16X3,
+           L.PH_EPI_NONE, None, None, 0, 1.0, 0.0, None, 0, 0, 0, D._stream())
+    ref = a[:K].double().t() @ b[:K].double()
+    assert ((out.double() - ref).norm() / ref.norm()).item() < 2.5 * 2 ** -17 + 1e-5

@@ -191,13 +191,53 @@ def test_tiled_scan_bit_exact(gpu, dt, B, T, time_major, variant):
     assert np.array_equal(r.cpu().numpy().ravel(), ref)
 
 
+@pytest.mark.parametrize("variant", [0, 1])
+@pytest.mark.parametrize("time_major", [True, False])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("B,T", [(20, 70), (9000, 40)])
+def test_tiled_scan_non_finite(gpu, dt, B, T, time_major, variant):
+    """NaN and infinite rewards, values, ratios and done flags travel through the tiles as through the sequential twin
+    (a terminal stops them; a step past the ends of a tile adds nothing of them)."""
+    rew, val, done, logr, boot = _bench_inputs(B, T, seed=0x4900)
+    ratio = np.exp(logr)
+    lay = lambda x: x.reshape((T, B) if time_major else (B, T))
+    for x, t, b, v in ((rew, 3, 1, np.nan), (rew, T - 1, 2, np.inf), (val, 10, 3, np.nan), (val, 0, 4, -np.inf),
+                       (val, T - 1, 5, np.nan), (ratio, 8, 6, np.nan), (ratio, 20, 7, np.inf), (done, 12, 8, np.nan),
+                       (rew, 30, B - 1, -np.inf), (val, 31, 0, np.inf)):
+        lay(x)[(t, b) if time_major else (b, t)] = v
+    for t, b in ((2, 1), (15, 3)):  # terminals before a NaN in the walk
+        lay(done)[(t, b) if time_major else (b, t)] = 1.0
+    ref, _ = O.vtrace(rew, val, done, ratio, boot, B, T, variant=variant, time_major=time_major, dtype=dt)
+    tt = torch.float32 if dt == np.float32 else torch.float64
+    c = lambda x: _cuda(x, tt).reshape((T, B) if time_major else (B, T))
+    adv, _ = D.vtrace(c(rew), c(val), c(done), c(ratio), _cuda(boot, tt), variant=variant, time_major=time_major)
+    assert np.array_equal(adv.cpu().numpy().ravel(), ref, equal_nan=True)
+    assert np.isnan(ref).any() and np.isfinite(ref).any()
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float64])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("n,at", [(1, 0), (300, 299), (4097, 4096), (20000, 5000)])
+def test_adv_normalize_non_finite(gpu, dt, bad, n, at):
+    """One non-finite value: the mean is it (NaN or infinite), the std NaN and every element NaN, as in two passes."""
+    x = torch.randn(n, generator=torch.Generator().manual_seed(n), dtype=torch.float64).to(dt)
+    x[at] = bad
+    stats = torch.zeros(2, device="cuda", dtype=dt)
+    y = D.adv_normalize(x.cuda(), stats=stats).cpu()
+    assert torch.isnan(y).all() and torch.isnan(stats[1]).item()
+    assert torch.equal(stats[:1].cpu().isnan(), x.mean().reshape(1).isnan())
+    if bad == bad:
+        assert stats[0].item() == bad
+
+
 @pytest.mark.parametrize("dt", [torch.float32, torch.float64])
 @pytest.mark.parametrize("n", [1, 2, 255, 4095, 4096, 4097, 8191, 70001])
 @pytest.mark.parametrize("mean", [0.0, 300.0])
 def test_adv_normalize_chunk_edges(gpu, dt, n, mean):
-    """Mean and std of one read in 4096-element chunks, moved to the common mean: against f64. The fp32 mean of
-    n values of size m is off by about m 2^-24 (chunk sums of 16 values per lane and trees), relative to a std of 1;
-    4e-5 covers m = 300 (4 x 300 x 2^-24 = 7e-5 at worst per chunk, averaged over chunks), 1e-12 f64."""
+    """Mean and std of one read in 4096-element chunks, moved to the common mean: against f64. A mean of values of size m
+    is off by a few m 2^-24 in fp32 (sums of 16 values per lane, then trees of 8 levels: 4 m 2^-24 = 7e-5 at m = 300,
+    relative to a std of 1): 8e-5 there and 1e-5 at m = 0, on the mean itself times m / 30, as it is compared
+    unscaled; f64 is 2^29 finer, and 1e-11 covers the division by std + 1e-8 as well."""
     x = torch.randn(n, generator=torch.Generator().manual_seed(n), dtype=torch.float64) + mean
     x = x.to(dt)
     stats = torch.zeros(2, device="cuda", dtype=dt)

@@ -908,7 +908,8 @@ int ns_small(float* const* X, const int* rows, const int* cols, int n, const flo
 }
 
 std::atomic<unsigned> g_spin{kSpinLimit};
-// 0: by shape (one workgroup per matrix, one XCD per matrix, or one device-wide queue); 1: always one device-wide queue; 2: one XCD per matrix whenever the device has 8 XCDs of 32 CUs
+// 0: by shape (one workgroup per matrix, one XCD per matrix, or one device-wide queue); 1: always one device-wide
+// queue; 2: one XCD per matrix whenever the device has 8 XCDs of 32 CUs
 std::atomic<int> g_queues{0};
 
 __global__ void k_clear_word(unsigned* w) {

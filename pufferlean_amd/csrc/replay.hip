@@ -97,8 +97,9 @@ __global__ void __launch_bounds__(256) k_seg_l1_sm(const R* __restrict__ adv, lo
 //   draw i: z = splitmix64 finaliser of rng + (i+1)*GOLD; u = (z >> 11) / 2^53 * total;
 //           idx = first e with cum[e] >= u (N-1 if none); mp[i] = exp(-beta * log(N * p[idx] + 1e-12))
 // Past a few segments and draws (prio_one_block) the f64 exponentials and logarithms of the weights and the draws
-// are what takes the time in one workgroup, so they are spread over the chip: a kernel of weights, then (N up to kPsLdsCum) blocks of kPsDraws draws that
-// each form the table from the weights in their LDS, the same operations in the same order in every block.
+// are what takes the time in one workgroup, so they are spread over the chip: a kernel of weights, then (N up to
+// kPsLdsCum) blocks of kPsDraws draws that each form the table from the weights in their LDS, the same
+// operations in the same order in every block.
 // 4096 segments, 4096 draws: 21.9 us in one workgroup, 10.1 in the two launches.
 __device__ __forceinline__ double prio_p(double w, double denom) { return (w + 1e-6) / denom; }
 

@@ -187,7 +187,8 @@ def release_scratch():
 
 def newton_schulz_batch(Xs, *, coeffs=CONST_COEFFS, eps=1e-7, math="bf16"):
     """In-place fast-tier NS of several independent fp32 matrices; equal to calling newton_schulz on
-    each. bf16: one fused launch per 16 matrices; fp32: concurrently on the library's stream lanes."""
+    each. bf16: one launch per 16 matrices (a workgroup each if all are small); fp32: one launch per phase
+    for 16 matrices, the largest shapes concurrently on the library's stream lanes."""
     _dev(*Xs)
     for X in Xs:
         if X.dtype != torch.float32 or not X.is_contiguous():

@@ -14,8 +14,9 @@
 // (count, mean, M2) partials; the normalising kernel's blocks merge them in block order (Chan et al.'s
 // pairwise update), so mean and std cost no extra pass over the columns. Segment-major columns pass
 // through LDS tiles of 16 segments x 64 steps, so that both the segment rows and the timestep-major
-// minibatch are read and written in runs. The iterate writes the last draw of a segment: found through a
-// last-writer table that the second launch leaves zeroed, or for long rows by comparing the draws in each block.
+// minibatch are read and written in runs. The iterate writes the last draw of a segment: found by comparing the
+// draws in each block, or for many draws and time-major columns through a last-writer table that the second
+// launch leaves zeroed.
 //
 // Every reduction here has a fixed order, so results are reproducible run to run. They are not
 // bit-identical to the CPU twins, whose sums are sequential: mean, std, the probability normaliser
@@ -180,13 +181,14 @@ __global__ void __launch_bounds__(kPsThreads) k_prio_draws(const double* __restr
   if (threadIdx.x < kPsDraws && i < B) prio_draw(i, cum, w, N, total, denom, beta, rng, seg, mp);
 }
 
-// prio_one_block: weights, table and draws in one launch of one workgroup, one segment per thread.
-constexpr long kPsOne = kPsThreads;
+// prio_one_block: weights, table and draws in one launch of one workgroup.
+constexpr long kPsOne = 2048;
 __global__ void __launch_bounds__(kPsThreads) k_prio_one(const double* __restrict__ L1, long N, long B, double alpha,
                                                          double beta, unsigned long long rng, int* __restrict__ seg,
                                                          double* __restrict__ mp) {
   __shared__ double red[kPsThreads];
   __shared__ double w[kPsOne], cum[kPsOne];
+  static_assert((kPsThreads + 2 * kPsOne) * 8 <= kMaxLdsBytes, "LDS budget");
   for (long e = threadIdx.x; e < N; e += kPsThreads) w[e] = prio_weight(L1[e], alpha);
   __syncthreads();
   double denom;
@@ -606,7 +608,7 @@ int prio_sample(const double* L1, size_t N, size_t B, double alpha, double beta,
   if (B == 0) return PH_OK;
   PH_REQUIRE(L1 && seg && mp, "prio_sample: null buffer");
   if (prio_one_block((long)N, (long)B)) {
-    static_assert(kPsOne >= 1024, "segments of prio_one_block");
+    static_assert(kPsOne >= 2048, "segments of prio_one_block");
     k_prio_one<<<1, kPsThreads, 0, st>>>(L1, (long)N, (long)B, alpha, beta, (unsigned long long)rng, seg, mp);
     PH_LAUNCH_CHECK();
     return PH_OK;

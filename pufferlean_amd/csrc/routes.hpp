@@ -79,21 +79,22 @@ inline bool seg_l1_tiled(bool f64, bool time_major, long N, long T) {
   return f64 ? T >= 32 : T >= 64 && N >= 128;
 }
 
-// The sampler in one workgroup: few segments and draws, whose f64 functions are quick and where a second launch costs
-// more than they do (64 segments, 64 draws 5.6 us in one launch, 6.7 in two; 1024, 512 7.4 / 8.2; but 1024, 2048
-// 10.6 / 8.1 and 2048, 1024 10.2 / 8.8).
-inline bool prio_one_block(long N, long draws) { return N <= 1024 && draws <= 1024; }
+// The sampler in one workgroup: few segments and draws, where a second launch (3.7 us of host time) costs more than
+// spreading the f64 functions saves (one launch / two: 64 segments, 64 draws 5.6 / 6.7 us, 1024 and 512 7.4 / 8.2, 2048 and
+// 512 9.2 / 8.7, 2048 and 1024 10.2 / 8.8; but 1024 and 2048 10.6 / 8.1, 3072 and 1024 11.7 / 9.2).
+inline bool prio_one_block(long N, long draws) { return N <= 2048 && draws <= 1024; }
 
 // The value / ratio iterate: tiles of 16 draws x 64 steps that compare their draws with every later one, in one launch,
 // or two launches through a last-writer table with a wavefront per draw. The comparison costs each block a pass
-// over the draws (so a bound on them), the table a launch; a wavefront per draw reads B apart in the timestep-major
-// inputs and is one chain over T. f64, table / tiles, over twenty sets of columns in turn (an update's columns are new
-// to the L2): 64 draws of 64 steps 4.1 / 5.2 us, 4096 of 16 6.0 / 7.0, 4096 of 32 7.1 / 7.5, 1024 of 64 5.7 / 5.7, 4096 of
-// 64 9.1 / 7.6, 256 of 128 5.9 / 5.4, 512 of 256 8.1 / 6.3, 4096 of 128 13.5 / 8.3; 16 of 1024 8.0 / 4.0. (The same set
-// again and again, the L2 warm: 4096 of 64 6.1 / 6.5, 1024 of 128 5.1 / 5.2, 4096 of 256 21.8 / 10.1.)
+// over the draws (so a bound on them), the table a launch (3.7 us of host time, which is what bounds a chain of such
+// calls issued one by one); a wavefront per draw reads B apart in the timestep-major inputs and is one chain over T.
+// f64, table / tiles, over twenty sets of columns in turn (an update's columns are new to the L2): 64 draws of 16 steps
+// 4.1 / 5.5 us, 4096 of 16 6.0 / 7.0, 4096 of 32 7.1 / 7.5, 1024 of 64 5.7 / 5.7, 4096 of 64 9.1 / 7.6, 512 of 256 8.1 /
+// 6.3, 4096 of 128 13.5 / 8.3; 8192 of 16 7.3 / 10.0, of 32 9.1 / 9.9, of 48 10.7 / 10.2; 16 of 1024 8.0 / 4.0. The
+// replay chain of 1363 segments x 71 steps and 100 draws issued one by one: 39.9 us with the table, 36.2 with the tiles.
 inline bool iterate_tiled(bool time_major, long draws, long T) {
-  if (time_major || draws > 8192 || T > 1L << 30) return false;
-  return T >= 256 || (T >= 128 && draws >= 256) || (T >= 64 && draws >= 1024);
+  if (time_major || T < 16 || T > 1L << 30) return false;
+  return draws <= 4096 || (draws <= 8192 && T >= 48);
 }
 
 // ---- Newton-Schulz in fp32 ----------------------------------------------------------------------------------

@@ -90,7 +90,8 @@ def test_iterate_more_draws_than_the_pairwise_scan(gpu):
 
 
 @pytest.mark.parametrize("N,T,B", [(60, 20, 8192), (60, 256, 8192), (60, 256, 8193), (300, 255, 40), (300, 257, 40),
-                                   (7, 130, 255), (3000, 128, 256), (50, 64, 1023), (50, 65, 1024), (50, 64, 8192), (5, 1000, 1)])
+                                   (7, 15, 100), (3000, 16, 255), (50, 47, 4096), (50, 47, 4097), (50, 48, 4097), (50, 64, 8192),
+                                   (5, 1000, 1)])
 def test_iterate_forms(gpu, N, T, B):
     """Both sides of the rule between the tiles that compare draws and the last-writer table: the last draw of a
     segment leaves its values, ratios to f64's exponential, other rows untouched; invalid draws are skipped."""
@@ -130,7 +131,7 @@ def test_gather_statistics_forms(gpu, T, B, time_major):
 
 
 @pytest.mark.parametrize("N,B", [(8192, 1), (8192, 129), (8193, 129), (1024, 128), (1025, 127), (1, 5), (63, 1024),
-                                 (1024, 1024), (1000, 1025)])
+                                 (1024, 1024), (1000, 1025), (2048, 1024), (2049, 1024), (1777, 600)])
 def test_sampler_edges(gpu, N, B):
     L1 = rng.randf(0x740 + N, N, 0.01, 5.0)
     seg, mp = D.prio_sample(torch.from_numpy(L1).cuda(), B, alpha=0.8, beta=0.2, rng_state=0x1234)

@@ -104,15 +104,14 @@ def test_gather_tiled(route, T, tiled):
     assert route("gather_tiled", 0, T) == tiled and route("gather_tiled", 1, T) == 0
 
 
-@pytest.mark.parametrize("N,draws,one", [(1, 1, 1), (64, 64, 1), (1024, 1024, 1), (1025, 64, 0), (64, 1025, 0), (1024, 2048, 0),
+@pytest.mark.parametrize("N,draws,one", [(1, 1, 1), (64, 64, 1), (1024, 1024, 1), (2048, 1024, 1), (2049, 64, 0), (64, 1025, 0), (1024, 2048, 0),
                                          (4096, 4096, 0)])
 def test_prio_one_block(route, N, draws, one):
     assert route("prio_one_block", N, draws) == one
 
 
-@pytest.mark.parametrize("draws,T,tiled", [(64, 16, 0), (64, 64, 0), (4096, 16, 0), (8192, 16, 0), (8192, 32, 0), (4096, 63, 0),
-                                           (1023, 64, 0), (1024, 64, 1), (4096, 64, 1), (8192, 64, 1), (255, 128, 0),
-                                           (256, 128, 1), (16, 256, 1), (4096, 256, 1), (8193, 256, 0)])
+@pytest.mark.parametrize("draws,T,tiled", [(64, 15, 0), (64, 16, 1), (4096, 16, 1), (4097, 47, 0), (4097, 48, 1), (8192, 16, 0),
+                                           (8192, 32, 0), (8192, 64, 1), (16, 1024, 1), (4096, 256, 1), (8193, 256, 0)])
 def test_iterate_tiled(route, draws, T, tiled):
     assert route("iterate_tiled", 0, draws, T) == tiled and route("iterate_tiled", 1, draws, T) == 0
 

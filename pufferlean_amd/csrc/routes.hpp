@@ -119,11 +119,12 @@ inline bool ns_f32_fits(int rows, int cols) {
 // (below 320 units 10 / 28 / 36; steps of two layers, 512 units: 512 rows 31 / 38 / 44 us, 700 44 / 40 / 45, 2048 71 /
 // 42 / 48, 4096 126 / 74 / 57, chain 88; 384: 1500 58 / 37 / 43, chain 46). Past 1280 units few rows go to the chain,
 // whose split k keeps the chip busy (2048 units, 48 rows 75, chain 60; 200 rows 128-row blocks 82, chain 100).
-// fp32 products, bound by the matrix core, 768 blocks of 32 rows or 256 of 128, a round of either about as long; 256-row
-// blocks are never the faster form. Past 512 units the chain's 128x128 tiles fill their rounds better at some
-// sizes (in units of a round: 9 per round of 128-row blocks + 3, 11 per round of chain tiles + 5.5; 768 units: 2600
-// rows 204, chain 264; 3300 294, chain 274), and past 768 the chain takes the few rows (896: 256 rows 92, chain 95; 300
-// 101, chain 95; 1024: 100 rows 100, chain 94, but 1024 rows in 128-row blocks 165, chain 203).
+// fp32 products, bound by the matrix core, 768 blocks of 32 rows or 256 of 128, the chain 256 tiles of 128x128; 256-row
+// blocks are never the faster form. Costs of r rounds: 10 r + 1, 8 r + 12 and 11 r + 14 (512 units: 1300 rows 79 / 94 us,
+// chain 128; 2048 104 / 95 / 131; 4096 170 / 152 / 201; 328 units, 7072 rows 163 in 128-row blocks, chain 158; 768: 2600
+// rows 243 / 204 / 264, 3300 293 / 294 / 274). A chain of less than two rounds is longer than its tiles say, its gaps
+// showing. Past 768 units the chain takes the few rows (896: 256 rows 92, chain 95; 300 101, chain 95; 1024: 100 rows 100, chain
+// 94, but 1024 rows in 128-row blocks 165, chain 203).
 enum RollForm { kRollChain = 0, kRoll32, kRoll128, kRoll256 };
 inline RollForm rollout_form(bool bf16, long N, long H) {
   const auto up = [](long a, long b) { return (a + b - 1) / b; };
@@ -137,10 +138,11 @@ inline RollForm rollout_form(bool bf16, long N, long H) {
   }
   if (H > 2048) return kRollChain;
   if (H > 768 && N <= 768) return H <= 896 && N <= 256 ? kRoll32 : kRollChain;
-  const long r32 = up(b32, 768), r128 = up(b128, 256), chain = up(up(N, 128) * up(3 * H, 128), 256);
-  if (H > 512 && (r128 >= 2 || H > 768) && 18 * r128 + 6 >= 22 * chain + 11) return kRollChain;
-  if (H > 768) return kRoll128;
-  return r32 <= r128 ? kRoll32 : kRoll128;
+  const long r32 = up(b32, 768), r128 = up(b128, 256), rc = up(up(N, 128) * up(3 * H, 128), 256);
+  if (H > 768) return 18 * r128 + 6 < 22 * rc + 11 ? kRoll128 : kRollChain;
+  const long c32 = 10 * r32 + 1, c128 = 8 * r128 + 12, chain = 11 * rc + 14;
+  if ((rc >= 2 || r128 >= 2) && chain <= c32 && chain <= c128) return kRollChain;
+  return c32 <= c128 ? kRoll32 : kRoll128;
 }
 
 }  // namespace ph

@@ -126,7 +126,7 @@ ROLLOUT = [(1, 48, 128, 1), (1, 2048, 128, 1), (1, 16384, 128, 3), (1, 4096, 256
            (1, 700, 512, 2), (1, 2048, 512, 2), (1, 2600, 512, 3), (1, 4096, 512, 3), (1, 1500, 384, 2), (1, 3300, 384, 3),
            (1, 1024, 640, 2), (1, 300, 1024, 2), (1, 2600, 768, 2), (1, 200, 1280, 2), (1, 48, 2048, 0), (1, 200, 2048, 2),
            (1, 48, 4096, 0), (0, 48, 128, 1), (0, 8192, 128, 2), (0, 2048, 384, 1), (0, 1300, 512, 1), (0, 2048, 512, 2),
-           (0, 4096, 512, 2), (0, 6000, 256, 1), (0, 4096, 640, 0), (0, 2600, 768, 2), (0, 3300, 768, 0), (0, 48, 896, 1),
+           (0, 4096, 512, 2), (0, 6000, 256, 1), (0, 4096, 640, 0), (0, 7072, 328, 0), (0, 2600, 768, 2), (0, 3300, 768, 0), (0, 48, 896, 1),
            (0, 300, 896, 0), (0, 700, 896, 0), (0, 1, 1024, 0), (0, 1024, 1024, 2), (0, 2600, 1024, 0), (0, 48, 2048, 0),
            (0, 2048, 1280, 0), (0, 1024, 2048, 2), (0, 1024, 2056, 0)]
 

@@ -50,14 +50,14 @@ inline int sample_registers(long A) {
 // 18.6 us against 26.1 tiled). Below that a lane is one chain of dependent load rounds that grows with T, and a
 // chunk costs the same whether its 64 steps are real or not: short horizons stay with the lanes (fp32 4096 segments,
 // lanes / tiles: T = 4 3.0 / 3.2 us, 8 3.4 / 3.3, 64 13.1 / 6.1; 16384, tiles of 64 segments: 16 5.0 / 5.7, 32 8.0 /
-// 6.6; f64 4096: 8 4.2 / 3.8, 8192: 8 4.3 / 4.5, 16384: 12 5.8 / 6.0), and where the two are close a chunk that is
-// mostly padding decides (fp32 32767 segments: 64 16.0 / 12.6, 72 16.9 / 17.6, 96 21.5 / 19.5).
-// Segment-major: lanes read T elements apart, so tiles win sooner (fp32 4096: 2 3.5 / 3.2, 4 5.3 / 3.3; 16384: 4 5.3 /
+// 6.6; f64 64: 8 3.4 / 3.7, 188: 11 4.5 / 3.9, 8192: 8 4.3 / 4.5, 16384: 12 5.8 / 6.0), and where the two are close a
+// chunk that is mostly padding decides (fp32 32767 segments: 64 16.0 / 12.6, 72 16.9 / 17.6, 96 21.5 / 19.5).
+// Segment-major: lanes read T elements apart, so tiles win sooner (fp32 64: 4 2.7 / 3.1; 4096: 4 5.3 / 3.3; 16384: 4 5.3 /
 // 6.0, 8 9.9 / 6.1; 65536: 8 10.8 / 12.1, 12 15.4 / 12.7; f64 256: 4 3.0 / 3.7, 8 5.9 / 3.8; 32767: 8 8.4 / 9.6).
 inline bool vtrace_tiled(bool f64, bool time_major, long B, long T) {
-  if (!time_major) return T >= (f64 ? (B <= 16384 ? 8 : 12) : (B <= 8192 ? 4 : B <= 32768 ? 8 : 12));
+  if (!time_major) return T >= (f64 ? (B <= 16384 ? 8 : 12) : (B > 128 && B <= 8192 ? 4 : B <= 32768 ? 8 : 12));
   const long pad = (T + 63) / 64 * 64 - T;
-  if (B <= 8192) return T >= (f64 ? 12 : 8);
+  if (B <= 8192) return T >= (f64 ? (B <= 4096 ? 10 : 12) : 8);
   if (f64) return B <= 16384 ? T >= 16 : B <= 24576 && 2 * pad <= T;
   return B <= 24576 ? T >= 32 : B < 32768 && 2 * pad <= T;
 }
@@ -123,8 +123,8 @@ inline bool ns_f32_fits(int rows, int cols) {
 // blocks are never the faster form. Costs of r rounds: 10 r + 1, 8 r + 12 and 11 r + 14 (512 units: 1300 rows 79 / 94 us,
 // chain 128; 2048 104 / 95 / 131; 4096 170 / 152 / 201; 328 units, 7072 rows 163 in 128-row blocks, chain 158; 768: 2600
 // rows 243 / 204 / 264, 3300 293 / 294 / 274). A chain of less than two rounds is longer than its tiles say, its gaps
-// showing. Past 768 units the chain takes the few rows (896: 256 rows 92, chain 95; 300 101, chain 95; 1024: 100 rows 100, chain
-// 94, but 1024 rows in 128-row blocks 165, chain 203).
+// showing. Past 768 units the chain takes the few rows (896: 256 rows 92, chain 95; 300 101, chain 95; 1024: 100 rows
+// 100, chain 94, but 1024 rows in 128-row blocks 165, chain 203).
 enum RollForm { kRollChain = 0, kRoll32, kRoll128, kRoll256 };
 inline RollForm rollout_form(bool bf16, long N, long H) {
   const auto up = [](long a, long b) { return (a + b - 1) / b; };

@@ -83,7 +83,7 @@ VTRACE = [(0, 1, 4096, 1, 0), (0, 1, 4096, 4, 0), (0, 1, 4096, 8, 1), (0, 1, 163
           (1, 1, 24576, 16, 0), (1, 1, 24576, 65, 0), (1, 1, 24576, 128, 1), (1, 1, 32767, 65, 0), (0, 0, 4096, 1, 0),
           (0, 0, 4096, 4, 1), (0, 0, 16384, 4, 0), (0, 0, 16384, 8, 1), (0, 0, 65536, 1, 0), (0, 0, 65536, 8, 0),
           (0, 0, 65536, 64, 1), (1, 0, 256, 4, 0), (1, 0, 4096, 8, 1), (1, 0, 32767, 8, 0), (1, 0, 65536, 2, 0),
-          (1, 0, 65536, 64, 1)]
+          (1, 0, 65536, 64, 1), (0, 0, 93, 5, 0), (0, 0, 129, 5, 1), (0, 0, 93, 8, 1), (1, 1, 188, 11, 1), (1, 1, 8192, 11, 0)]
 
 
 @pytest.mark.parametrize("f64,tm,B,T,tiled", VTRACE)

@@ -107,7 +107,7 @@ __global__ void __launch_bounds__(256) k_ppo_grad_md(const float* __restrict__ o
 // and the stride, the block's rows are one run of floats and move with 16-byte loads and stores. Each lane works on
 // its row in LDS, so a block holds only its rows (250007x15: 19 KB); registers bound the blocks per CU (four or
 // five), whose load, compute and store phases overlap. Loops over a head's columns are unrolled with an exit at
-// the head's size, which is the same for every lane; heads past 12 columns take one pass of 16 or 32 masked ones,
+// the head's size, which is the same for every lane; heads past 12 columns take one pass of 16, 24 or 32 masked ones,
 // whose exponentials run side by side (one head of 31, 4096 rows: 24.6 us with exits, 16.3 masked; heads of 9 and 5
 // at 250007 rows 27.0 masked, 20 with exits). 4096 rows at a stride of 32: heads 9 and 5 15.4 -> 12.8 us.
 constexpr int kTileW = 32;
@@ -580,7 +580,8 @@ int ppo_grad_md(const float* out, size_t ldo, const int* act, const float* adv, 
           out, (long)ldo, act, adv, ret, old, ov, (long)N, hs, W, vf, ent, clip, vfClip, dout, (long)ldd,
           linear_rows(out, ldo, W + 1), linear_rows(dout, ldd, W + 1), newlp, newval, part, losses);
     };
-    if (widest > 16) go(std::integral_constant<int, 32>{});
+    if (widest > 24) go(std::integral_constant<int, 32>{});
+    else if (widest > 16) go(std::integral_constant<int, 24>{});
     else if (widest > 12) go(std::integral_constant<int, 16>{});
     else go(std::integral_constant<int, 0>{});
   } else

@@ -37,7 +37,7 @@ LAYOUTS = ["packed", "strided", "offset"]
 
 @pytest.mark.parametrize("N", [1, 63, 255, 256, 257, 1001])
 @pytest.mark.parametrize("sizes", [[1], [2], [9, 5], [3, 3, 4, 1], [31], [1, 2, 3, 4, 5, 6, 7, 3], [12, 7, 3],
-                                   [13, 2], [16, 15], [17, 1]])
+                                   [13, 2], [16, 15], [17, 1], [24, 3], [25]])
 def test_md_tile(gpu, N, sizes):
     K, W = len(sizes), sum(sizes)
     out = f32(rng.normal(0xB01 + N, N * (W + 1)).reshape(N, W + 1) * 2.0)
